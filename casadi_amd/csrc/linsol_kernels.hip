@@ -17,6 +17,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstdlib>
 #include <cstring>
 #include <map>
 #include <memory>
@@ -26,6 +27,7 @@
 
 #include "../../include/casadi_hip.h"
 #include "capi_common.hpp"
+#include "linsol_rows.hpp"
 #include "tape_internal.hpp"
 
 using namespace sxh;
@@ -399,6 +401,8 @@ struct cxh_ldl_s {
   std::map<int, std::shared_ptr<sxh::LinsolJit>> jit;  // specialised factor + solve per nrhs
   std::shared_ptr<sxh::LinsolJit> jit_fact;            // specialised factor alone
   std::shared_ptr<sxh::LinsolJit> jit_solve;  // specialised solve alone, one right-hand side
+  std::unique_ptr<sxh::RowsProgram> rows[3];           // sixteen lanes per instance, per LinsolPart
+  bool rows_tried[3] = {false, false, false};          // rows[part] null afterwards: the pattern does not fit
   int64_t fact_n = -1;                                 // instances factored by the last nfact (-1: none)
 };
 
@@ -414,6 +418,8 @@ struct cxh_qr_s {
   std::map<int, std::shared_ptr<sxh::LinsolJit>> jit;  // specialised factor + solve per (nrhs, tr)
   std::shared_ptr<sxh::LinsolJit> jit_fact;            // specialised factor alone
   std::shared_ptr<sxh::LinsolJit> jit_solve[2];  // specialised solve alone, one right-hand side, per tr
+  std::unique_ptr<sxh::RowsProgram> rows[2];           // sixteen lanes per instance: fused, factor alone
+  bool rows_tried[2] = {false, false};                 // rows[part] null afterwards: the pattern does not fit
   int64_t fact_n = -1;                                 // instances factored by the last nfact (-1: none)
   // factorisations remembered (LinsolQr's "cache" option): each holds a copy
   // of the batch of A values it was computed from, and its V, R, beta
@@ -426,6 +432,84 @@ struct cxh_qr_s {
   std::vector<int> cache_loc;  // most recently used first; -1: never filled
   DeviceBuffer cmp_flag;
 };
+
+// Largest batch of the sixteen-lane programs (CXH_LINSOL_ROWS_MAX overrides).
+// They spend about four times the instructions of the one-lane programs per
+// instance on four times the wavefronts: ahead while the one-lane programs
+// leave SIMDs idle, behind once those fill the chip.  Horizon-30 KKT, us per
+// call, sixteen-lane / one-lane: LDL 141 / 333 at 8192 instances, 285 / 434 at
+// 16384, 573 / 585 at 32768, 877 / 772 at 49152; QR 271 / 805, 602 / 927,
+// 1132 / 1251, 1613 / 1558.
+static int64_t rows_max() {
+  if (const char* e = std::getenv("CXH_LINSOL_ROWS_MAX")) return std::atoll(e);
+  return 32768;
+}
+
+// 32-bit byte strides and offsets: a row of n_inst doubles, the kept blocks.
+static bool rows_fit(const sxh::RowsProgram& P, int64_t n_inst) {
+  const int64_t n16 = round_up(n_inst, 64);
+  return n16 * 8 < (int64_t(1) << 32) && n16 * P.kept * 8 < (int64_t(1) << 32);
+}
+
+static sxh::RowsProgram* ldl_rows_program(cxh_ldl_s* l, int part) {
+  if (!l->rows_tried[part]) {
+    l->rows_tried[part] = true;
+    auto P = std::make_unique<sxh::RowsProgram>();
+    if (sxh::rows_ldl_source(l->lt.ncol, l->a.colind, l->a.row, l->lt.colind, l->lt.row, l->p, part, *P))
+      l->rows[part] = std::move(P);
+  }
+  return l->rows[part].get();
+}
+
+// The sixteen-lane program that serves a call, compiled; null: the one-lane
+// programs serve it.
+static sxh::RowsProgram* ldl_rows(cxh_ldl_s* l, int part, int64_t n_inst) {
+  if (n_inst > rows_max()) return nullptr;
+  sxh::RowsProgram* P = ldl_rows_program(l, part);
+  if (P && !rows_fit(*P, n_inst)) return nullptr;
+  if (P && !sxh::rows_ready(*P)) {
+    l->rows[part].reset();
+    P = nullptr;
+  }
+  return P;
+}
+
+static sxh::RowsProgram* qr_rows_program(cxh_qr_s* q, int part) {
+  if (!q->rows_tried[part]) {
+    q->rows_tried[part] = true;
+    auto P = std::make_unique<sxh::RowsProgram>();
+    if (sxh::rows_qr_source(q->a.ncol, q->v.nrow, q->a.colind, q->a.row, q->v.colind, q->v.row, q->r.colind, q->r.row,
+                            q->prinv, q->pc, part, *P))
+      q->rows[part] = std::move(P);
+  }
+  return q->rows[part].get();
+}
+
+static sxh::RowsProgram* qr_rows(cxh_qr_s* q, int part, int64_t n_inst) {
+  if (n_inst > rows_max()) return nullptr;
+  sxh::RowsProgram* P = qr_rows_program(q, part);
+  if (P && !rows_fit(*P, n_inst)) return nullptr;
+  if (P && !sxh::rows_ready(*P)) {
+    q->rows[part].reset();
+    P = nullptr;
+  }
+  return P;
+}
+
+// Source and index table of a sixteen-lane program (length 0: none).
+static int rows_text(const sxh::RowsProgram* P, char* buf, int64_t cap, int64_t* len, int32_t* tab, int64_t tab_cap,
+                     int64_t* tab_len) {
+  const int64_t n = P ? static_cast<int64_t>(P->source.size()) : 0, m = P ? static_cast<int64_t>(P->tab.size()) : 0;
+  if (len) *len = n;
+  if (tab_len) *tab_len = m;
+  if (buf && cap > 0) {
+    const size_t k = static_cast<size_t>(std::min(n, cap - 1));
+    if (k) std::memcpy(buf, P->source.data(), k);
+    buf[k] = '\0';
+  }
+  if (tab && m) std::memcpy(tab, P->tab.data(), static_cast<size_t>(std::min(m, tab_cap)) * sizeof(int32_t));
+  return 0;
+}
 
 static sxh::LinsolJit& qr_program(cxh_qr_s* q, int nrhs, bool tr) {
   auto& J = q->jit[2 * nrhs + (tr ? 1 : 0)];
@@ -542,9 +626,24 @@ int cxh_ldl_factor_solve(cxh_ldl l, int64_t n_inst, const double* a, double* x, 
   const int64_t nnz_a = l->a.colind.back();
   l->fact_n = -1;  // the fused call keeps no factors
   if (l->engine == CXH_ENGINE_JIT) {
+    const bool soa = layout == CXH_SOA;
+    if (sxh::RowsProgram* R = nrhs == 1 ? ldl_rows(l, LS_FUSED, n_inst) : nullptr) {
+      sxh::RowsIO io;
+      io.ld = round_up(n_inst, 64);
+      l->w.reserve(static_cast<size_t>(R->kept * round_up(n_inst, 16)) * sizeof(double));
+      io.a = a;
+      io.a_s = soa ? n_inst : 1;
+      io.a_t = soa ? 1 : nnz_a;
+      io.x = x;
+      io.x_s = soa ? n_inst : 1;
+      io.x_t = soa ? 1 : n;
+      io.w = l->w.as<double>();
+      io.status = status;
+      sxh::rows_launch(*R, n_inst, io, static_cast<hipStream_t>(stream));
+      return 0;
+    }
     auto& J = l->jit[nrhs];
     if (!J) J = jit_ldl_create(n, l->a.colind, l->a.row, l->lt.colind, l->lt.row, l->p, nrhs);
-    const bool soa = layout == CXH_SOA;
     return jit_linsol_run(*J, n_inst, a, soa ? n_inst : 1, soa ? 1 : nnz_a, x, soa ? n_inst : 1,
                        soa ? 1 : static_cast<int64_t>(n) * nrhs, status, static_cast<hipStream_t>(stream));
   }
@@ -566,13 +665,26 @@ int cxh_ldl_nfact(cxh_ldl l, int64_t n_inst, const double* a, int32_t* status, i
   const int64_t nnz_a = l->a.colind.back(), nnz_lt = l->lt.colind.back();
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (l->engine == CXH_ENGINE_JIT) {
-    if (!l->jit_fact) l->jit_fact = jit_ldl_create(n, l->a.colind, l->a.row, l->lt.colind, l->lt.row, l->p, 0,
-                                                   LS_FACTOR);
     const int64_t ld = round_up(n_inst, 64);
     l->lt_vals.reserve(std::max<size_t>(nnz_lt, 1) * ld * sizeof(double));
     l->d_vals.reserve(std::max<size_t>(n, 1) * ld * sizeof(double));
     double* fac[2] = {l->lt_vals.as<double>(), l->d_vals.as<double>()};
     const bool soa = layout == CXH_SOA;
+    if (sxh::RowsProgram* R = ldl_rows(l, LS_FACTOR, n_inst)) {
+      sxh::RowsIO io;
+      io.ld = ld;
+      io.a = a;
+      io.a_s = soa ? n_inst : 1;
+      io.a_t = soa ? 1 : nnz_a;
+      io.f = fac[0];
+      io.d = fac[1];
+      io.status = status;
+      sxh::rows_launch(*R, n_inst, io, s);
+      l->fact_n = n_inst;
+      return 0;
+    }
+    if (!l->jit_fact) l->jit_fact = jit_ldl_create(n, l->a.colind, l->a.row, l->lt.colind, l->lt.row, l->p, 0,
+                                                   LS_FACTOR);
     if (int rc = jit_linsol_factor(*l->jit_fact, n_inst, a, soa ? n_inst : 1, soa ? 1 : nnz_a, fac, 2, ld, status, s))
       return rc;
   } else {
@@ -596,11 +708,26 @@ int cxh_ldl_solve(cxh_ldl l, int64_t n_inst, double* x, int32_t nrhs, int32_t tr
   const int n = l->lt.ncol;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (l->engine == CXH_ENGINE_JIT) {
-    auto& J = l->jit_solve;
-    if (!J) J = jit_ldl_create(n, l->a.colind, l->a.row, l->lt.colind, l->lt.row, l->p, 1, LS_SOLVE);
     const int64_t ld = round_up(n_inst, 64);
     const double* fac[2] = {l->lt_vals.as<double>(), l->d_vals.as<double>()};
     const bool soa = layout == CXH_SOA;
+    if (sxh::RowsProgram* R = ldl_rows(l, LS_SOLVE, n_inst)) {
+      sxh::RowsIO io;
+      io.ld = ld;
+      l->w.reserve(static_cast<size_t>(R->kept * round_up(n_inst, 16)) * sizeof(double));
+      io.x_s = soa ? n_inst : 1;
+      io.x_t = soa ? 1 : static_cast<int64_t>(n) * nrhs;
+      io.f = l->lt_vals.as<double>();
+      io.d = l->d_vals.as<double>();
+      io.w = l->w.as<double>();
+      for (int q = 0; q < nrhs; ++q) {
+        io.x = x + static_cast<int64_t>(q) * n * io.x_s;
+        sxh::rows_launch(*R, n_inst, io, s);
+      }
+      return 0;
+    }
+    auto& J = l->jit_solve;
+    if (!J) J = jit_ldl_create(n, l->a.colind, l->a.row, l->lt.colind, l->lt.row, l->p, 1, LS_SOLVE);
     // the right-hand sides one after another: each is solved on its own, in
     // the order the fused program solves it, so the bits are the same
     for (int q = 0; q < nrhs; ++q)
@@ -654,6 +781,24 @@ int cxh_ldl_jit_source(cxh_ldl l, int32_t nrhs, char* buf, int64_t cap, int64_t*
     buf[m] = '\0';
   }
   return 0;
+  CXH_CATCH
+}
+
+int cxh_ldl_rows_source(cxh_ldl l, int32_t part, char* buf, int64_t cap, int64_t* len, int32_t* tab, int64_t tab_cap,
+                        int64_t* tab_len) {
+  CXH_TRY
+  if (!l) return cxh_fail("null ldl handle");
+  if (part < LS_FUSED || part > LS_SOLVE) return cxh_fail("cxh_ldl_rows_source: part must be 0, 1 or 2");
+  return rows_text(ldl_rows_program(l, part), buf, cap, len, tab, tab_cap, tab_len);
+  CXH_CATCH
+}
+
+int cxh_qr_rows_source(cxh_qr q, int32_t part, char* buf, int64_t cap, int64_t* len, int32_t* tab, int64_t tab_cap,
+                       int64_t* tab_len) {
+  CXH_TRY
+  if (!q) return cxh_fail("null qr handle");
+  if (part < LS_FUSED || part > LS_FACTOR) return cxh_fail("cxh_qr_rows_source: part must be 0 or 1");
+  return rows_text(qr_rows_program(q, part), buf, cap, len, tab, tab_cap, tab_len);
   CXH_CATCH
 }
 
@@ -807,6 +952,22 @@ int cxh_qr_factor_solve(cxh_qr q, int64_t n_inst, const double* a, double* x, in
   q->fact_n = -1;  // the fused call keeps no factors
   if (q->engine == CXH_ENGINE_JIT) {
     const bool soa = layout == CXH_SOA;
+    if (sxh::RowsProgram* R = nrhs == 1 && !tr ? qr_rows(q, LS_FUSED, n_inst) : nullptr) {
+      sxh::RowsIO io;
+      io.ld = round_up(n_inst, 64);
+      q->w.reserve(static_cast<size_t>(R->kept * round_up(n_inst, 16)) * sizeof(double));
+      io.a = a;
+      io.a_s = soa ? n_inst : 1;
+      io.a_t = soa ? 1 : nnz_a;
+      io.x = x;
+      io.x_s = soa ? n_inst : 1;
+      io.x_t = soa ? 1 : ncol;
+      io.w = q->w.as<double>();
+      io.status = status;
+      io.eps = q->eps;
+      sxh::rows_launch(*R, n_inst, io, static_cast<hipStream_t>(stream));
+      return 0;
+    }
     return jit_linsol_run(qr_program(q, nrhs, tr != 0), n_inst, a, soa ? n_inst : 1, soa ? 1 : nnz_a, x,
                           soa ? n_inst : 1, soa ? 1 : static_cast<int64_t>(ncol) * nrhs, status,
                           static_cast<hipStream_t>(stream));
@@ -895,16 +1056,30 @@ int cxh_qr_nfact(cxh_qr q, int64_t n_inst, const double* a, int32_t* status, int
     st = nullity.as<int32_t>();
   }
   if (q->engine == CXH_ENGINE_JIT) {
-    if (!q->jit_fact)
-      q->jit_fact = jit_qr_create(q->a.ncol, q->v.nrow, q->a.colind, q->a.row, q->v.colind, q->v.row, q->r.colind,
-                                  q->r.row, q->prinv, q->pc, q->eps, 0, false, LS_FACTOR);
     q->v_vals.reserve(bv);
     q->r_vals.reserve(br);
     q->beta.reserve(bb);
     double* fac[3] = {q->v_vals.as<double>(), q->r_vals.as<double>(), q->beta.as<double>()};
     const bool soa = layout == CXH_SOA;
+    if (sxh::RowsProgram* R = qr_rows(q, LS_FACTOR, n_inst)) {
+      sxh::RowsIO io;
+      io.ld = ld;
+      io.a = a;
+      io.a_s = soa ? n_inst : 1;
+      io.a_t = soa ? 1 : nnz_a;
+      io.z = fac[0];
+      io.f = fac[1];
+      io.d = fac[2];
+      io.status = st;
+      io.eps = q->eps;
+      sxh::rows_launch(*R, n_inst, io, s);
+    } else {
+    if (!q->jit_fact)
+      q->jit_fact = jit_qr_create(q->a.ncol, q->v.nrow, q->a.colind, q->a.row, q->v.colind, q->v.row, q->r.colind,
+                                  q->r.row, q->prinv, q->pc, q->eps, 0, false, LS_FACTOR);
     if (int rc = jit_linsol_factor(*q->jit_fact, n_inst, a, soa ? n_inst : 1, soa ? 1 : nnz_a, fac, 3, ld, st, s))
       return rc;
+    }
   } else {
     qr_generic(q, LS_FACTOR, n_inst, a, nullptr, 0, 0, st, layout, s);
   }

@@ -110,6 +110,21 @@ class Linsol:
                                     C.byref(ns)), "cxh_qr_jit_source")
         return buf.value.decode(), ns.value
 
+    def rows_source(self, part=0):
+        """Generated source and index table of the sixteen-lanes-per-instance
+        program (part 0: factor + solve, 1: factor alone, 2: LDL solve alone),
+        or None when the pattern does not fit that form."""
+        fn = L.cxh_ldl_rows_source if self.solver == "ldl" else L.cxh_qr_rows_source
+        n, m = L.I64(), L.I64()
+        L.check(fn(self._h, int(part), None, 0, C.byref(n), None, 0, C.byref(m)), fn.__name__)
+        if n.value == 0:
+            return None
+        buf = C.create_string_buffer(n.value + 1)
+        tab = np.zeros(m.value, np.int32)
+        L.check(fn(self._h, int(part), buf, n.value + 1, C.byref(n), tab.ctypes.data_as(C.POINTER(L.I32)), m.value,
+                   C.byref(m)), fn.__name__)
+        return buf.value.decode(), tab
+
     def name(self):
         return self._name
 

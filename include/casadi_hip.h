@@ -468,6 +468,11 @@ int cxh_ldl_rank(cxh_ldl l, int32_t* rank, void* stream);
 int cxh_ldl_engine(cxh_ldl l, int32_t engine);
 /* Introspection: generated source of the specialised kernel for nrhs.     */
 int cxh_ldl_jit_source(cxh_ldl l, int32_t nrhs, char* buf, int64_t cap, int64_t* len);
+/* Generated source and index table of the sixteen-lanes-per-instance program
+ * (part 0: factor + solve of one right-hand side, 1: factor alone, 2: solve
+ * alone); both lengths are 0 when the pattern does not fit that form. */
+int cxh_ldl_rows_source(cxh_ldl l, int32_t part, char* buf, int64_t cap, int64_t* len, int32_t* tab,
+                        int64_t tab_cap, int64_t* tab_len);
 
 /* Batched sparse Householder QR (casadi_qr / casadi_qr_solve,
  * casadi/core/runtime/casadi_qr.hpp:53-200, LinsolQr
@@ -509,6 +514,9 @@ int cxh_qr_engine(cxh_qr q, int32_t engine);
  * kernels for (nrhs, tr), with the number of segments.                      */
 int cxh_qr_jit_source(cxh_qr q, int32_t nrhs, int32_t tr, int32_t segment, char* buf, int64_t cap,
                       int64_t* len, int32_t* n_segments);
+/* The same for the QR (parts 0 and 1; not transposed). */
+int cxh_qr_rows_source(cxh_qr q, int32_t part, char* buf, int64_t cap, int64_t* len, int32_t* tab,
+                       int64_t tab_cap, int64_t* tab_len);
 
 /* Facts of the current device: compute units, LDS per compute unit in KiB,
  * the device name (truncated to name_len).  Replaces nothing in the
