@@ -59,6 +59,7 @@
 #include "sx_ops.h"
 #include "tape_internal.hpp"
 #include "jit_common.hpp"
+#include "jit_parts.hpp"
 
 namespace sxh {
 
@@ -96,6 +97,8 @@ struct CxjArgs {
 #define CXJ_KEEP_PTR(x) asm volatile("" : "+s"(x))
 #define CXJ_AFTER(p, x) asm volatile("" : "+s"(p) : "v"(x))
 #define CXJ_GLOBAL __attribute__((address_space(1)))
+#define CXJ_LDS __attribute__((address_space(3)))
+#define CXJ_TABLE __attribute__((address_space(4)))
 #define CXJ_OPAQUE(p) asm volatile("" : "+v"(p))
 #define CXJ_OPAQUE_AFTER(p, x) asm volatile("" : "+v"(p) : "v"(x))
 #endif
@@ -1417,7 +1420,7 @@ static int jac_dir_group(int ndir, int64_t n) {
 }
 
 static JitJac& jac_plan(cxh_jac_s* j, int64_t n) {
-  const int want = j->ndir == 0 ? 1 : std::min(std::max(j->ndir, 1), std::min(jac_dir_group(j->ndir, n), 64));
+  const int want = j->ndir == 0 ? 1 : j->dir_group > 0 ? std::min(j->dir_group, std::max(j->ndir, 1)) : std::min(std::max(j->ndir, 1), std::min(jac_dir_group(j->ndir, n), 64));
   if (j->jit && j->jit->group == want) return *j->jit;
   const cxh_tape_s* t = j->tape;
   auto J = std::make_shared<JitJac>();
@@ -1563,7 +1566,24 @@ static int jac_prefetch(const cxh_jac_s* j) {
 //
 // State and spill rows are tiled [group][instance/64][row][64]: a row's offset
 // is a compile-time constant and accesses of a wave are 512 B contiguous.
-static std::string gen_tangent(const cxh_jac_s* j, const JitJac& J, int g, int s, int R, int* spill_rows) {
+//
+// part: the plan is a class of independent parts (PartClass), number `cls` of
+// its kernel.  A row that advances by a fixed step from part to part (stages
+// of a horizon) is computed from the part's number, any other comes from the
+// row table: a scalar load waited for at every use (245 of them
+// in the quadrotor stage's program).
+static std::string gen_tangent(const cxh_jac_s* j, const JitJac& J, int g, int s, int R, int* spill_rows,
+                               const PartClass* part = nullptr, int cls = 0) {
+  auto row = [&](int k) {
+    if (!part) return std::to_string(k);
+    const int* r = part->rows->data() + part->first_row + k;
+    const int len = part->row_len(), step = part->count > 1 ? r[len] - r[0] : 0;
+    for (int p = 1; p < part->count; ++p)
+      if (r[static_cast<int64_t>(p) * len] != r[0] + p * step) return "cxj_rows[" + std::to_string(k) + "]";
+    return step == 0 ? std::to_string(r[0]) : "(" + std::to_string(r[0]) + " + cxj_part * " + std::to_string(step) + ")";
+  };
+  auto out_row = [&](int k) { return row(part ? part->n_in + k : k); };
+  auto jac_row = [&](int q) { return row(part ? part->n_in + part->n_out + q : q); };
   const cxh_tape_s* t = j->tape;
   const int nd = j->ndir;
   const int d0 = g * J.group, d1 = std::min(nd, d0 + J.group);
@@ -1785,7 +1805,7 @@ static std::string gen_tangent(const cxh_jac_s* j, const JitJac& J, int g, int s
   // accesses of one row.
   auto opaque = [&](const char* base, bool is_const, const std::string& after) {
     const std::string p = "cxj_p" + std::to_string(n_ptr++);
-    b += std::string("  CXJ_GLOBAL ") + (is_const ? "const " : "") + "double* " + p + " = " + base + ";\n";
+    b += std::string(part && std::strcmp(base, "cxj_ss") == 0 ? "  CXJ_SPILL " : "  CXJ_GLOBAL ") + (is_const ? "const " : "") + "double* " + p + " = " + base + ";\n";
     b += after.empty() ? "  CXJ_OPAQUE(" + p + ");\n" : "  CXJ_OPAQUE_AFTER(" + p + ", " + after + ");\n";
     return p;
   };
@@ -1852,7 +1872,7 @@ static std::string gen_tangent(const cxh_jac_s* j, const JitJac& J, int g, int s
         load = ptr(p_in, "cxj_si") + "[" + std::to_string(64 * v.in_row) + "]";
       } else if (v.kind == 2) {
         use_arg.insert(v.ai);
-        load = ptr(p_arg[v.ai], "cxj_a" + std::to_string(v.ai)) + "[" + std::to_string(v.aj) + " * A.arg.a[" +
+        load = ptr(p_arg[v.ai], "cxj_a" + std::to_string(v.ai)) + "[" + row(v.aj) + " * A.arg.a[" +
                std::to_string(v.ai) + "].s_nz]";
       } else {
         throw std::logic_error("tangent codegen: value neither resident nor stored");
@@ -1863,7 +1883,12 @@ static std::string gen_tangent(const cxh_jac_s* j, const JitJac& J, int g, int s
       res.insert({next_use(v), id});
     }
   };
-  char buf[256];
+  if (part) {  // the inputs come from far away (HBM) and are few: all at once, ahead of everything
+    std::vector<int> in;
+    for (size_t v = 0; v < val.size(); ++v)
+      if (val[v].kind == 2 && !val[v].uses.empty()) in.push_back(static_cast<int>(v));
+    if (static_cast<int>(in.size()) <= R / 2) reload(in);
+  }
   for (size_t i = 0; i < ops.size(); ++i) {
     const Op& op = ops[i];
     const int ii = static_cast<int>(i);
@@ -1900,15 +1925,14 @@ static std::string gen_tangent(const cxh_jac_s* j, const JitJac& J, int g, int s
       const std::string ks = std::to_string(op.k);
       if (e.op == OP_OUTPUT) {
         if (g == 0) {
-          std::snprintf(buf, sizeof buf, "  CXJ_OUT(%d, %d, %s);\n", e.i0, e.i2, val[op.x].name.c_str());
-          b += buf;
+          b += "  CXJ_OUT(" + std::to_string(e.i0) + ", " + out_row(e.i2) + ", " + val[op.x].name + ");\n";
         }
         const int64_t flat = j->out_off[e.i0] + e.i2;
         for (int d = d0; d < d1; ++d) {
           const int2 tg = j->scatter[flat * nd + d];
           const std::string v = op.tx[d - d0] >= 0 ? val[op.tx[d - d0]].name : std::string("0.0");
-          if (tg.x >= 0) b += "  CXJ_SENS(0, " + std::to_string(tg.x) + ", " + v + ");\n";
-          if (tg.y >= 0) b += "  CXJ_SENS(0, " + std::to_string(tg.y) + ", " + v + ");\n";
+          if (tg.x >= 0) b += "  CXJ_SENS(0, " + jac_row(tg.x) + ", " + v + ");\n";
+          if (tg.y >= 0) b += "  CXJ_SENS(0, " + jac_row(tg.y) + ", " + v + ");\n";
         }
       } else {
         const std::string& X = val[op.x].name;
@@ -1978,18 +2002,26 @@ static std::string gen_tangent(const cxh_jac_s* j, const JitJac& J, int g, int s
   const std::string gs = std::to_string(g);
   std::string o;
   o.reserve(b.size() + 1024);
-  o += "__device__ __forceinline__ void cxj_body_g" + gs + "(const CxjArgs& A, const long long k) {\n"
-       "  const long long cxj_tb = (k >> 6) * (CXJ_TROWS * 64LL) + (k & 63) + " + gs + "LL * A.lds * CXJ_TROWS;\n"
-       "  const long long cxj_sb = (k >> 6) * (CXJ_SROWS * 64LL) + (k & 63) + " + gs + "LL * A.lds * CXJ_SROWS;\n";
-  if (use_si) o += "  CXJ_GLOBAL const double* const cxj_si = (CXJ_GLOBAL const double*)A.st_in + cxj_tb;\n";
-  if (use_so) o += "  CXJ_GLOBAL double* const cxj_so = (CXJ_GLOBAL double*)A.st_out + cxj_tb;\n";
-  if (use_ss) o += "  CXJ_GLOBAL double* const cxj_ss = (CXJ_GLOBAL double*)A.spill + cxj_sb;\n";
+  if (part) {  // one segment: no state rows; the spill rows tiled [class, part, group][instance/64][row][64] or in LDS
+    o += "__device__ __forceinline__ void cxj_body_c" + std::to_string(cls) + "_g" + gs +
+         "(const CxjArgs& A, const long long k, const int cxj_unit, const int cxj_part, const CXJ_TABLE int* const "
+         "cxj_rows) {\n";
+    if (use_ss) o += "  CXJ_SPILL double* const cxj_ss = CXJ_SPILL_BASE(cxj_unit);\n";
+    o += "  (void)cxj_unit;\n  (void)cxj_part;\n  (void)cxj_rows;\n";
+  } else {
+    o += "__device__ __forceinline__ void cxj_body_g" + gs + "(const CxjArgs& A, const long long k) {\n"
+         "  const long long cxj_tb = (k >> 6) * (CXJ_TROWS * 64LL) + (k & 63) + " + gs + "LL * A.lds * CXJ_TROWS;\n"
+         "  const long long cxj_sb = (k >> 6) * (CXJ_SROWS * 64LL) + (k & 63) + " + gs + "LL * A.lds * CXJ_SROWS;\n";
+    if (use_si) o += "  CXJ_GLOBAL const double* const cxj_si = (CXJ_GLOBAL const double*)A.st_in + cxj_tb;\n";
+    if (use_so) o += "  CXJ_GLOBAL double* const cxj_so = (CXJ_GLOBAL double*)A.st_out + cxj_tb;\n";
+    if (use_ss) o += "  CXJ_GLOBAL double* const cxj_ss = (CXJ_GLOBAL double*)A.spill + cxj_sb;\n";
+    o += "  (void)cxj_tb;\n  (void)cxj_sb;\n";
+  }
   for (int i : use_arg) {
     const std::string is = std::to_string(i);
     o += "  CXJ_GLOBAL const double* const cxj_a" + is + " = (CXJ_GLOBAL const double*)A.arg.a[" + is +
          "].p + k * A.arg.a[" + is + "].s_inst;\n";
   }
-  o += "  (void)cxj_tb;\n  (void)cxj_sb;\n";
   o += b;
   o += "}\n";
   return o;
@@ -2010,7 +2042,8 @@ static std::string gen_tangent_kernel(const cxh_jac_s* j, const JitJac& J, int s
   std::string o = kSxOpsSource;
   o += kPrologue;
   o.reserve(o.size() + bodies.size() + 1024);
-  o += "#define CXJ_TROWS " + std::to_string(J.home_rows) + "\n#define CXJ_SROWS " + std::to_string(sp) + "\n";
+  o += "#define CXJ_TROWS " + std::to_string(J.home_rows) + "\n#define CXJ_SROWS " + std::to_string(sp) +
+       "\n";
   o += bodies;
   o += "__device__ __forceinline__ void cxj_body(const CxjArgs& A, const long long k, const int grp) {\n"
        "  switch (grp) {\n";
@@ -2024,8 +2057,172 @@ static std::string gen_tangent_kernel(const cxh_jac_s* j, const JitJac& J, int s
   return finish_source(std::move(o));
 }
 
+// ---- independent parts (jit_parts.hip)
+//
+// One kernel: blockIdx.y counts the units (class, part, direction group), the
+// class with the most work first.
+struct JitParts {
+  std::vector<std::unique_ptr<PartClass>> cls;  // empty: the tape does not split
+  std::vector<int> rows;
+  DeviceBuffer d_rows, spill, zero;
+  struct Kernel {
+    hipFunction_t fn = nullptr;
+    int64_t units = 0, spill_rows = 0;  // spill rows in device memory (0: in LDS, or none)
+  };
+  std::map<std::array<int, 3>, Kernel> fn;  // by (directions per group, 32-bit offsets, outputs stored)
+};
+
+// Spill rows a block of 64 lanes keeps in LDS: 40 KB, so that four blocks
+// (one wavefront per SIMD) share a CU's 160 KB.
+constexpr int kPartLdsRows = 80;
+
+// outs: whether the outputs are stored (all of them or none).
+static std::string gen_parts_kernel(JitParts& P, int R, int group, bool soa32, bool outs, int* n_units, int* spill_rows) {
+  std::string bodies, dispatch;
+  int sp = 0, unit = 0;
+  for (size_t c = 0; c < P.cls.size(); ++c) {
+    PartClass& C = *P.cls[c];
+    C.jac.dir_group = group;
+    const JitJac& J = jac_plan(&C.jac, 0);
+    if (J.n_seg != 1) throw std::logic_error("parts: a class of more than one segment");
+    for (int g = 0; g < J.n_group; ++g) {
+      int ns = 0;
+      bodies += gen_tangent(&C.jac, J, g, 0, R, &ns, &C, static_cast<int>(c));
+      sp = std::max(sp, ns);
+    }
+    const std::string u0 = std::to_string(unit), ng = std::to_string(J.n_group), cs = std::to_string(c);
+    unit += C.count * J.n_group;
+    dispatch += "  if (u < " + std::to_string(unit) + ") {\n    const int part = (u - " + u0 + ") / " + ng +
+                ";\n    const CXJ_TABLE int* const rows = (const CXJ_TABLE int*)A.adj_in + " + std::to_string(C.first_row) +
+                " + part * " + std::to_string(C.row_len()) + ";\n    switch ((u - " + u0 + ") % " + ng + ") {\n";
+    for (int g = 0; g < J.n_group; ++g)
+      dispatch += "      case " + std::to_string(g) + ": cxj_body_c" + cs + "_g" + std::to_string(g) + "(A, k, u, part, rows); break;\n";
+    dispatch += "    }\n    return;\n  }\n";
+  }
+  const bool lds = sp > 0 && sp <= kPartLdsRows;
+  *n_units = unit;
+  *spill_rows = lds ? 0 : sp;
+  std::string o = soa32 ? "#define CXJ_SOA32\n" : "";
+  o += kSxOpsSource;
+  o += kPrologue;
+  o.reserve(o.size() + bodies.size() + 4096);
+  // the blocks are known to be there or not: no branch around a store (each
+  // would end a basic block)
+  o += std::string("#undef CXJ_SENS\n#define CXJ_SENS(i, j, v) *const_cast<double*>(CXJ_AT(A.asens, i, j)) = (v)\n#undef CXJ_OUT\n") +
+       (outs ? "#define CXJ_OUT(i, j, v) *const_cast<double*>(CXJ_AT(A.res, i, j)) = (v)\n" : "#define CXJ_OUT(i, j, v) ((void)0)\n");
+  if (lds) {
+    o += "__shared__ double cxj_lds[" + std::to_string(sp * 64) + "];\n#define CXJ_SPILL CXJ_LDS\n"
+         "#define CXJ_SPILL_BASE(u) ((CXJ_LDS double*)cxj_lds + threadIdx.x)\n";
+  } else {
+    o += "#define CXJ_SROWS " + std::to_string(sp) + "\n#define CXJ_SPILL CXJ_GLOBAL\n"
+         "#define CXJ_SPILL_BASE(u) ((CXJ_GLOBAL double*)A.spill + (k >> 6) * (CXJ_SROWS * 64LL) + (k & 63) + (u) * A.lds * "
+         "CXJ_SROWS)\n";
+  }
+  o += bodies;
+  o += "extern \"C\" __global__ void __launch_bounds__(64) cxj_parts(const CxjArgs A) {\n"
+       "  const long long k = (long long)blockIdx.x * 64 + threadIdx.x;\n"
+       "  if (k >= A.n) return;\n"
+       "  const int u = (int)blockIdx.y;\n" + dispatch + "}\n";
+  return finish_source(std::move(o));
+}
+
+static bool parts_enabled() {
+  const char* e = std::getenv("CXH_JIT_PARTS");
+  return !(e && e[0] == '0') && !std::getenv("CXH_JIT_TANSEG");
+}
+
+// Directions per group of the parts' programs: each group computes the primal
+// again, and each direction more needs more values resident.  Quadrotor
+// Hessian (10 directions, horizon 20), us at 16384 / 1001 / 64 instances:
+// 3 directions 275 / 29 / 14 (49 spill rows, in LDS), 2: 294 / 26 / 14, 1: 465 /
+// 45 / 21, 5: 345 / 43 / 30 (135 spill rows, in device memory).  Register
+// budgets of 100-120 values (two wavefronts per SIMD) spill to device memory
+// as well: 470-530 us.
+static int parts_dir_group() {
+  if (const char* e = std::getenv("CXH_JIT_DIRGROUP")) return std::max(1, std::atoi(e));
+  return 3;
+}
+
+static int parts_reg_budget() {
+  if (const char* e = std::getenv("CXH_JIT_TANREGS")) return std::max(8, std::atoi(e));
+  return 200;
+}
+
+static JitParts& parts_of(cxh_jac_s* j) {
+  if (!j->parts) {
+    j->parts = std::make_shared<JitParts>();
+    j->parts->cls = find_parts(j, j->parts->rows);
+    for (auto& c : j->parts->cls) c->rows = &j->parts->rows;
+  }
+  return *j->parts;
+}
+
+static bool all_soa(const IOTable& t, size_t n) {
+  for (size_t i = 0; i < n; ++i)
+    if (t.a[i].p && t.a[i].s_inst != 1) return false;
+  return true;
+}
+
+// The sweep over the parts of the tape; false when it does not split (or the
+// kernel would need scratch) and the whole tape's kernels serve the call.
+static bool parts_map_jac(cxh_jac_s* j, int64_t n, CxjArgs A, hipStream_t s) {
+  if (!parts_enabled() || j->ndir == 0) return false;
+  int have = 0, blocks = 0;  // output blocks given
+  for (size_t i = 0; i < j->tape->nnz_out.size(); ++i)
+    if (j->tape->nnz_out[i] > 0) {
+      ++blocks;
+      have += A.res.a[i].p != nullptr;
+    }
+  if (!A.asens.a[0].p || (have != 0 && have != blocks)) return false;
+  JitParts& P = parts_of(j);
+  if (P.cls.empty()) return false;
+  const int group = parts_dir_group();
+  const bool soa = static_cast<uint64_t>(n) * 8u < (uint64_t(1) << 32) && A.asens.a[0].s_inst == 1 &&
+                   all_soa(A.arg, j->tape->nnz_in.size()) && all_soa(A.res, j->tape->nnz_out.size());
+  JitParts::Kernel& K = P.fn[{group, soa ? 1 : 0, have ? 1 : 0}];
+  for (int R = parts_reg_budget(); !K.fn; R -= 24) {
+    if (R < 24) {
+      P.cls.clear();
+      return false;
+    }
+    int units = 0, ns = 0;
+    hipFunction_t f = jit_function(gen_parts_kernel(P, R, group, soa, have != 0, &units, &ns), "cxj_parts");
+    if (scratch_bytes(f) > 0) continue;
+    K.fn = f;
+    K.units = units;
+    K.spill_rows = ns;
+  }
+  if (K.units > 65535) return false;
+  if (!P.d_rows.ptr) P.d_rows.upload(P.rows.data(), P.rows.size() * sizeof(int));
+  if (K.spill_rows > 0) P.spill.reserve(static_cast<size_t>(K.spill_rows * K.units * A.lds) * sizeof(double));
+  for (auto& a : A.arg.a)  // an absent input reads zeros: one device zero, strides 0
+    if (!a.p) {
+      if (!P.zero.ptr) {
+        static const double zeros[8] = {};
+        P.zero.upload(zeros, sizeof zeros);
+      }
+      a = {P.zero.as<double>(), 0, 0};
+    }
+  A.adj_in = P.d_rows.as<double>();  // the row table
+  A.spill = K.spill_rows > 0 ? P.spill.as<double>() : nullptr;
+  void* params[] = {&A};
+  hip_check(hipModuleLaunchKernel(K.fn, static_cast<unsigned>((n + 63) / 64), static_cast<unsigned>(K.units), 1, 64, 1, 1, 0,
+                                  s, params, nullptr),
+            "jit parts kernel launch");
+  return true;
+}
+
 int jit_map_jac(cxh_jac_s* j, int64_t n, const IOTable& arg, const IOTable& res, double* jac, int64_t jac_s_nz,
                 int64_t jac_s_inst, hipStream_t s) {
+  if (j->ndir > 0 && (!j->parts || !j->parts->cls.empty())) {
+    CxjArgs A{};
+    A.arg = arg;
+    A.res = res;
+    A.asens.a[0] = {jac, jac_s_nz, jac_s_inst};
+    A.n = n;
+    A.lds = round_up(n, 64);
+    if (parts_map_jac(j, n, A, s)) return 0;
+  }
   JitJac& J = jac_plan(j, n);
   for (int sg = 0; sg < J.n_seg; ++sg) {
     hipFunction_t& f = J.fn[sg];
@@ -2075,6 +2272,16 @@ int jit_map_jac(cxh_jac_s* j, int64_t n, const IOTable& arg, const IOTable& res,
               "jit tangent kernel launch");
   }
   return 0;
+}
+
+// Source, row table and launch units of the parts' kernel ("" when the tape
+// does not split).
+std::string jit_parts_source(cxh_jac_s* j, bool soa32, int* n_units, int* spill_rows, std::vector<int>* rows) {
+  *n_units = *spill_rows = 0;
+  JitParts& P = parts_of(j);
+  if (P.cls.empty()) return "";
+  *rows = P.rows;
+  return gen_parts_kernel(P, parts_reg_budget(), parts_dir_group(), soa32, true, n_units, spill_rows);
 }
 
 std::string jit_tangent_source(cxh_jac_s* j, int s, int* n_group, int* n_seg) {
@@ -3455,6 +3662,27 @@ int cxh_jac_jit_source(cxh_jac j, int32_t segment, char* buf, int64_t cap, int64
   const std::string src = jit_tangent_source(j, segment, &ng, &ns);
   if (n_groups) *n_groups = ng;
   if (n_segments) *n_segments = ns;
+  if (len) *len = static_cast<int64_t>(src.size());
+  if (buf && cap > 0) {
+    const size_t m = std::min<size_t>(src.size(), static_cast<size_t>(cap - 1));
+    std::memcpy(buf, src.data(), m);
+    buf[m] = '\0';
+  }
+  return 0;
+  CXH_CATCH
+}
+
+int cxh_jac_parts_source(cxh_jac j, int32_t soa32, char* buf, int64_t cap, int64_t* len, int32_t* rows, int64_t rows_cap,
+                         int64_t* n_rows, int32_t* n_units, int32_t* spill_rows) {
+  CXH_TRY
+  if (!j) return cxh_fail("null jac plan");
+  int nu = 0, sp = 0;
+  std::vector<int> r;
+  const std::string src = jit_parts_source(j, soa32 != 0, &nu, &sp, &r);
+  if (n_units) *n_units = nu;
+  if (spill_rows) *spill_rows = sp;
+  if (n_rows) *n_rows = static_cast<int64_t>(r.size());
+  if (rows && !r.empty()) std::memcpy(rows, r.data(), sizeof(int32_t) * static_cast<size_t>(std::min<int64_t>(rows_cap, r.size())));
   if (len) *len = static_cast<int64_t>(src.size());
   if (buf && cap > 0) {
     const size_t m = std::min<size_t>(src.size(), static_cast<size_t>(cap - 1));

@@ -164,6 +164,7 @@ int roll_adj(cxh_tape_s* t, int mode, int64_t n, const IOTable& arg, const IOTab
 
 namespace sxh {
 struct JitJac;
+struct JitParts;
 }
 
 struct cxh_jac_s {
@@ -175,8 +176,10 @@ struct cxh_jac_s {
   std::vector<int2> scatter;    // [flat_out_nz][ndir] -> up to two Jacobian nonzeros
   sxh::DeviceBuffer d_seed, d_scatter, d_in_off, d_out_off;
   std::shared_ptr<sxh::JitJac> jit;  // specialised tangent kernels (jit.hip)
+  std::shared_ptr<sxh::JitParts> parts;  // the same over independent parts of the tape (jit.hip), once looked for
   int64_t seg_len = 0;               // instructions per kernel of the tangent sweep (0: default)
   int reg_budget = 0;                // starting register budget of its kernels (0: default)
+  int dir_group = 0;                 // directions per group (0: chosen from the batch)
   int prefetch = -1;                 // reload lookahead in instructions (-1: default)
   const char* kernel = "cxj_tan";    // name of its kernels (profiles tell the programs apart)
 };

@@ -568,6 +568,21 @@ class HipJacobian:
                                      C.byref(ns)), "cxh_jac_jit_source")
         return buf.value.decode(), ng.value, ns.value
 
+    def parts_source(self, soa32=False):
+        """Source of the kernel over the tape's independent parts, its row
+        table, launch units and spill rows, or None when it does not split."""
+        n, m, nu, sp = L.I64(), L.I64(), L.I32(), L.I32()
+        L.check(L.cxh_jac_parts_source(self._h, int(soa32), None, 0, C.byref(n), None, 0, C.byref(m), C.byref(nu),
+                                       C.byref(sp)), "cxh_jac_parts_source")
+        if n.value == 0:
+            return None
+        buf = C.create_string_buffer(n.value + 1)
+        rows = np.zeros(m.value, np.int32)
+        L.check(L.cxh_jac_parts_source(self._h, int(soa32), buf, n.value + 1, C.byref(n),
+                                       rows.ctypes.data_as(C.POINTER(L.I32)), m.value, C.byref(m), C.byref(nu),
+                                       C.byref(sp)), "cxh_jac_parts_source")
+        return buf.value.decode(), rows, nu.value, sp.value
+
     def __call__(self, args, n=None, res=True, stream=None):
         torch = _torch()
         like = self.tape._like(args)

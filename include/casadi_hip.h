@@ -227,6 +227,12 @@ int cxh_tape_roll_source(cxh_tape t, int64_t checkpoint_every, int32_t mode, cha
  * kernels when the plan's tape uses CXH_ENGINE_JIT.                         */
 int cxh_jac_jit_source(cxh_jac j, int32_t segment, char* buf, int64_t cap, int64_t* len,
                        int32_t* n_groups, int32_t* n_segments);
+/* Source of the kernel that runs the plan over the independent parts of its
+ * tape (soa32: 32-bit instance offsets), its row table, the launch's units
+ * (blockIdx.y) and spill rows per unit in device memory.  Length 0 when the
+ * tape does not split into repeated parts. */
+int cxh_jac_parts_source(cxh_jac j, int32_t soa32, char* buf, int64_t cap, int64_t* len, int32_t* rows,
+                         int64_t rows_cap, int64_t* n_rows, int32_t* n_units, int32_t* spill_rows);
 /* Compile a generated source for arch (e.g. "gfx950") without loading it;
  * 0 when it compiles, the compiler log in cxh_last_error otherwise.        */
 int cxh_jit_compile_check(const char* src, const char* arch);
