@@ -107,9 +107,9 @@ struct CxjArgs {
 #define CXJ_ANY(b) (__builtin_amdgcn_ballot_w64(b) != 0)
 #endif
 #ifdef CXJ_TRIG_CALLS
-#define CXJ_SINCOS(x_, s_, c_) do { const sxh::SinCos r_ = sxh::sxh_sincos_call(x_); s_ = r_.s; c_ = r_.c; } while (0)
+#define CXJ_SINCOS(x_, s_, c_, ...) do { const sxh::SinCos r_ = sxh::sxh_sincos_call(x_); s_ = r_.s; c_ = r_.c; } while (0)
 #else
-#define CXJ_SINCOS(x_, s_, c_) sxh::sxh_sincos(x_, &s_, &c_)
+#define CXJ_SINCOS(x_, s_, c_, ...) sxh::sxh_sincos(x_, &s_, &c_, ##__VA_ARGS__)
 #endif
 )CXJ";
 
@@ -377,6 +377,54 @@ bool fast_div_enabled() {
   return !(e && e[0] == '0');
 }
 
+// The quotient of two 53-bit integer significands X / Y is never midway between
+// two doubles, and x yh + RN(x yl) is within 2^-104 of it relatively (yl within
+// 2^-53 of 1 / c - yh, itself below 2^-52 / |c|, and as much again for the
+// rounding of x yl).  With X >= Y the midpoints are M / 2^53 for odd M in
+// (2^53, 2^54), at the distance |r| / (2^53 Y), r = 2^53 X - M Y: the sum can
+// round to the other side only where |r| <= 2^-51 X < 4.  With X < Y they are
+// M / 2^54, and |r| < 8 likewise.  M Y = -r modulo 2^53 (2^54) leaves few X
+// for each r, which are tried.
+bool div_pair(double c, double* yh, double* yl) {
+  using U = unsigned __int128;
+  int ex;
+  const double y = std::fabs(std::frexp(c, &ex)) * 2.0;  // [1, 2)
+  double h = 1.0 / y;
+  if (std::fma(-h, y, 1.0) < 0.0) h = std::nextafter(h, 0.0);
+  const double l = std::fma(-h, y, 1.0) / y;
+  const uint64_t Y = static_cast<uint64_t>(std::ldexp(y, 52));
+  int j = 0;
+  while (!((Y >> j) & 1)) ++j;
+  const uint64_t Yo = Y >> j;
+  uint64_t inv = Yo;  // Yo^-1 modulo 2^64 (Newton, 3 bits to start with)
+  for (int i = 0; i < 5; ++i) inv *= 2 - Yo * inv;
+  for (int sc = 53; sc <= 54; ++sc)
+    for (int64_t r = sc == 53 ? -4 : -8; r <= (sc == 53 ? 4 : 8); ++r) {
+      if (r == 0 || j >= sc || r % (int64_t(1) << j) != 0) continue;
+      const uint64_t mod = uint64_t(1) << (sc - j);
+      const uint64_t m0 = (static_cast<uint64_t>(-(r / (int64_t(1) << j))) * inv) & (mod - 1);
+      for (uint64_t M = m0 + (((uint64_t(1) << 53) - std::min(m0, uint64_t(1) << 53)) / mod) * mod; M < (uint64_t(1) << 54);
+           M += mod) {
+        if (M <= (uint64_t(1) << 53) || !(M & 1)) continue;
+        const U P = static_cast<U>(M) * Y + static_cast<U>(static_cast<__int128>(r));
+        const uint64_t X = static_cast<uint64_t>(P >> sc);
+        if ((static_cast<U>(X) << sc) != P || X < (uint64_t(1) << 52) || X >= (uint64_t(1) << 53)) continue;
+        if ((X >= Y) != (sc == 53)) continue;
+        const double x = std::ldexp(static_cast<double>(X), -52);
+        if (std::fma(x, h, x * l) != x / y) return false;
+      }
+    }
+  *yh = std::copysign(std::ldexp(h, 1 - ex), c);
+  *yl = std::copysign(std::ldexp(l, 1 - ex), c);
+  return true;
+}
+
+std::string div_c_call(const std::string& x, double c) {
+  double yh, yl;
+  if (div_pair(c, &yh, &yl)) return "sxh::sxh_div_c(" + x + ", " + lit(c) + ", " + lit(yh) + ", " + lit(yl) + ", wide)";
+  return "sxh::sxh_div_c(" + x + ", " + lit(c) + ", " + lit(1.0 / c) + ", wide)";
+}
+
 std::string lit(double d) {
   if (std::isnan(d)) return "__builtin_nan(\"\")";
   if (std::isinf(d)) return d > 0 ? "__builtin_huge_val()" : "(-__builtin_huge_val())";
@@ -428,14 +476,47 @@ static std::string adj_name(int64_t c, int64_t ws) {
 // boundary states, and the outputs of every sub-block but the last), 2 = the
 // rest, with the last sub-block reloaded from its stored state as well.  The
 // two halves of consecutive segments then run side by side (jit_adj).
+//
+// div (a single segment swept in one piece): divide by constants through
+// sxh_div_c and take sin/cos without a branch, hold every output and
+// sensitivity back to the end (an output may be written over an input), and
+// evaluate again with `<name>_x`, which divides as IEEE 754 does and calls the
+// library's sincos past 2^20, when a lane of the wavefront reported an operand
+// outside their ranges; *div counts the divisions and pairs.  The body is bound
+// by the instructions it issues (with few instances, by its chain), and an IEEE division is
+// eleven of them against four: the map of a cart-pole RK4 step (12
+// divisions, 4 pairs) over 8388608 instances 155.7 -> 130 us, the summed map's
+// gradient over 1048576 44.4 -> 41.7, a mixed batch of 77000 12.3 -> 11.6.
 static std::string gen_body(const cxh_tape_s* t, const JitPlan& P, int s, bool rev, const std::string& name,
-                            bool sub_blocks = true, int phase = 0, bool home = false) {
+                            bool sub_blocks = true, int phase = 0, bool home = false, int* div = nullptr) {
   const int t0 = P.t0[s], t1 = P.t0[s + 1];
   const int len = t1 - t0;
   const int64_t ws = t->ws;
   std::string o;
   o.reserve(static_cast<size_t>(len) * (rev ? 220 : 64) + 1024);
   o += "__device__ __forceinline__ void " + name + "(const CxjArgs& A, const long long k) {\n";
+  std::string held;  // the stores held back
+  int n_held = 0;
+  if (div) o += "  sxh::WaveFlag wide;\n";
+  // A held-back value is computed here: left to itself the compiler moves its
+  // last operations behind the branch, and their operands live until there.
+  auto store = [&](const std::string& macro, int i, int r, const std::string& v) {
+    const std::string at = "  " + macro + "(" + std::to_string(i) + ", " + std::to_string(r) + ", ";
+    if (!div) {
+      o += at + v + ");\n";
+      return;
+    }
+    const std::string h = "cxj_h" + std::to_string(n_held++);
+    o += "  double " + h + " = " + v + ";\n  CXJ_KEEP(" + h + ");\n";
+    held += at + h + ");\n";
+  };
+  auto finish = [&]() {
+    if (div)
+      o += "  if (__builtin_expect(CXJ_ANY(wide.any()), 0)) {\n    long long k2 = k;\n    CXJ_OPAQUE(k2);\n    " + name +
+           "_x(A, k2);\n    return;\n  }\n" + held;
+    o += "}\n";
+    return o;
+  };
   std::vector<int64_t> cur(ws, 0);
   const std::vector<int>& lin = P.live[s];
   const std::vector<int>& lout = P.live[s + 1];
@@ -522,6 +603,7 @@ static std::string gen_body(const cxh_tape_s* t, const JitPlan& P, int s, bool r
   // all_trig: every SIN / COS through sincos (the reverse sweep of this range
   // reads the complementary value as its partial); else only pairs
   auto emit_fwd = [&](int a, int b, int pass, bool outputs, bool all_trig = false) {
+    all_trig |= div != nullptr;
     const std::unordered_set<int64_t> pairs = all_trig ? std::unordered_set<int64_t>{} : trig_pairs(a, b, pass);
     for (int k = a; k < b; ++k) {
       const Instr& e = t->alg[k];
@@ -543,7 +625,9 @@ static std::string gen_body(const cxh_tape_s* t, const JitPlan& P, int s, bool r
             o += "  const double ts" + id + " = CXJ_SNAP(" + trig_ptr + ", " + std::to_string(r) + "), tc" + id +
                  " = CXJ_SNAP(" + trig_ptr + ", " + std::to_string(r + 1) + ");\n";
           } else {
-            o += "  double ts" + id + ", tc" + id + ";\n  CXJ_SINCOS(" + V(x) + ", ts" + id + ", tc" + id + ");\n";
+            o += "  double ts" + id + ", tc" + id + ";\n  CXJ_SINCOS(" + V(x) + ", ts" + id + ", tc" + id +
+                 (div ? ", wide);\n" : ");\n");
+            if (div) ++*div;
           }
           if (trig_io == 1) {
             const int64_t r = (*trig_counter)++;
@@ -571,8 +655,7 @@ static std::string gen_body(const cxh_tape_s* t, const JitPlan& P, int s, bool r
         case OP_OUTPUT:
           ox[k - t0] = cur[e.i1];
           if (outputs) {
-            std::snprintf(buf, sizeof buf, "  CXJ_OUT(%d, %d, %s);\n", e.i0, e.i2, V(cur[e.i1]).c_str());
-            o += buf;
+            store("CXJ_OUT", e.i0, e.i2, V(cur[e.i1]));
           }
           break;
         default: {
@@ -580,9 +663,15 @@ static std::string gen_body(const cxh_tape_s* t, const JitPlan& P, int s, bool r
           const int64_t y = op_is_binary(e.op) ? cur[e.i2] : x;
           ox[k - t0] = x;
           oy[k - t0] = y;
-          std::snprintf(buf, sizeof buf, "  const double %s = sxh::op_fun_full(%d, %s, %s);\n", nm.c_str(), e.op,
-                        V(x).c_str(), V(y).c_str());
-          o += buf;
+          if (div && e.op == OP_DIV && y >= 0 && (y & 3) < 2 && t->alg[y >> 2].op == OP_CONST &&
+              fast_divisor(t->alg[y >> 2].d)) {
+            o += "  const double " + nm + " = " + div_c_call(V(x), t->alg[y >> 2].d) + ";\n";
+            ++*div;
+          } else {
+            std::snprintf(buf, sizeof buf, "  const double %s = sxh::op_fun_full(%d, %s, %s);\n", nm.c_str(), e.op,
+                          V(x).c_str(), V(y).c_str());
+            o += buf;
+          }
           cur[e.i0] = vc[k - t0] = code;
         }
       }
@@ -594,8 +683,7 @@ static std::string gen_body(const cxh_tape_s* t, const JitPlan& P, int s, bool r
       for (size_t r = 0; r < lout.size(); ++r)
         if (P.fresh[s + 1][r])
           o += "  CXJ_ST_OUT(" + std::to_string(P.home[s + 1][r]) + ") = " + V(cur[lout[r]]) + ";\n";
-    o += "}\n";
-    return o;
+    return finish();
   }
   if (!rev) {
     emit_fwd(t0, t1, 0, true);
@@ -630,8 +718,7 @@ static std::string gen_body(const cxh_tape_s* t, const JitPlan& P, int s, bool r
         i += m;
       }
     }
-    o += "}\n";
-    return o;
+    return finish();
   }
   // sub-block boundaries and the live slots there
   const std::vector<int> c = sub_blocks ? sub_bounds(t0, t1) : std::vector<int>{t0, t1};
@@ -753,9 +840,7 @@ static std::string gen_body(const cxh_tape_s* t, const JitPlan& P, int s, bool r
           break;
         case OP_INPUT: {
           const int64_t v = vc[k - t0];
-          std::snprintf(buf, sizeof buf, "  CXJ_SENS(%d, %d, %s);\n", e.i1, e.i2,
-                        decl.count(v) ? Adj(v).c_str() : "0.0");
-          o += buf;
+          store("CXJ_SENS", e.i1, e.i2, decl.count(v) ? Adj(v) : std::string("0.0"));
           break;
         }
         default: {
@@ -789,21 +874,53 @@ static std::string gen_body(const cxh_tape_s* t, const JitPlan& P, int s, bool r
     }
   if (s == 0)
     for (const int2& u : t->unused_in) {
-      std::snprintf(buf, sizeof buf, "  CXJ_SENS(%d, %d, 0.0);\n", u.x, u.y);
-      o += buf;
+      store("CXJ_SENS", u.x, u.y, "0.0");
     }
-  o += "}\n";
-  return o;
+  return finish();
+}
+
+// Outputs (and, in a reverse sweep, sensitivities) a body may hold back for
+// its flagged divisions and sin/cos: past these the registers they keep cost
+// occupancy.  Over 2^20 instances of m outputs sin(a) / c + a^2 / d of 8 inputs,
+// held back against IEEE division (us): evaluation m = 8 24.9 / 27.3,
+// 16 39.4 / 47.9, 24 55.2 / 72.3, 32 94.1 / 99.7; reverse m + 8 = 12 29.6 / 30.1,
+// 16 42.3 / 42.5, 24 120 / 86.5.  The batch kernel, which has few wavefronts
+// anyway, gains up to the larger number: cart-pole, quadrotor and arm sweeps over 40000,
+// 12000 and 25000 instances 11.6 us with all three held back, 12.2 with only the
+// first, ten times as many 59.3 against 61.7 with none.
+constexpr int64_t kHeldEval = 32, kHeldReverse = 16;
+
+// gen_body of a tape that is one segment swept in one piece, with its divisions
+// by constants and sin/cos flagged (see gen_body) where that pays: the exact body
+// behind it is cold, so its sin/cos sites do not count towards trig_call_sites().
+static std::string gen_whole_body(const cxh_tape_s* t, const JitPlan& P, bool rev, const std::string& name, bool sub_blocks,
+                                  bool home, bool fast) {
+  int64_t held = 0;
+  for (const Instr& e : t->alg) held += e.op == OP_OUTPUT || (rev && e.op == OP_INPUT);
+  if (rev) held += static_cast<int64_t>(t->unused_in.size());
+  const bool one = P.n_seg == 1 && !(rev && sub_blocks && sub_bounds(P.t0[0], P.t0[1]).size() > 2);
+  if (fast && one && held <= (rev && sub_blocks ? kHeldReverse : kHeldEval) && fast_div_enabled()) {
+    int nd = 0;
+    const std::string f = gen_body(t, P, 0, rev, name, sub_blocks, 0, home, &nd);
+    if (nd > 0) {
+      std::string x = gen_body(t, P, 0, rev, name + "_x", sub_blocks, 0, home);
+      const std::string site = "  CXJ_SINCOS(";
+      for (size_t p = x.find(site); p != std::string::npos; p = x.find(site, p)) x.replace(p, site.size(), "\n CXJ_SINCOS(");
+      return x + f;
+    }
+  }
+  return gen_body(t, P, 0, rev, name, sub_blocks, 0, home);
 }
 
 // One segment kernel: one lane per instance, the arguments by value.  phase
 // (reverse kernels): 0 whole, 1 first pass (cxj_snap), 2 the rest.
 static std::string gen_segment(const cxh_tape_s* t, const JitPlan& P, int s, bool rev, int phase = 0,
-                               bool soa32 = false, bool home = false) {
+                               bool soa32 = false, bool home = false, bool fast = true) {
   std::string o = soa32 ? "#define CXJ_SOA32\n" : "";
   o += kSxOpsSource;
   o += kPrologue;
-  o += gen_body(t, P, s, rev, "cxj_body", true, rev ? phase : 0, home && !rev);
+  o += P.n_seg == 1 && !(rev && phase) ? gen_whole_body(t, P, rev, "cxj_body", true, home && !rev, fast)
+                                       : gen_body(t, P, s, rev, "cxj_body", true, rev ? phase : 0, home && !rev);
   if (rev || P.ipt == 1) {
     o += std::string("extern \"C\" __global__ void __launch_bounds__(256) ") +
          (rev ? (phase == 1 ? "cxj_snap" : "cxj_rev") : "cxj_fwd") +
@@ -921,13 +1038,25 @@ hipFunction_t jit_function_checked(const std::string& src, const char* name, con
   return f;
 }
 
+// The kernel of gen(true), whose divisions by constants hold stores back, or of
+// gen(false) where that needs scratch.
+static hipFunction_t fast_or_plain(const std::function<std::string(bool)>& gen, const char* name, const char* remedy) {
+  const std::string fast = gen(true), plain = gen(false);
+  if (fast != plain) {
+    hipFunction_t f = jit_function(fast, name);
+    if (scratch_bytes(f) == 0) return f;
+  }
+  return jit_function_checked(plain, name, remedy);
+}
+
 static hipFunction_t segment_kernel(cxh_tape_s* t, JitPlan& P, int s, bool rev) {
   hipFunction_t& f = rev ? P.rev[s] : P.fwd[s];
   if (!f)
-    f = jit_function_checked(gen_segment(t, P, s, rev), rev ? "cxj_rev" : "cxj_fwd",
-                             rev ? "use sub-blocks of at most 256 instructions (CXH_JIT_SUBBLOCK), a shorter "
-                                   "checkpoint interval or the interpreter engine"
-                                 : "use a shorter checkpoint interval or the interpreter engine");
+    f = fast_or_plain([&](bool fast) { return gen_segment(t, P, s, rev, 0, false, false, fast); },
+                      rev ? "cxj_rev" : "cxj_fwd",
+                      rev ? "use sub-blocks of at most 256 instructions (CXH_JIT_SUBBLOCK), a shorter "
+                            "checkpoint interval or the interpreter engine"
+                          : "use a shorter checkpoint interval or the interpreter engine");
   return f;
 }
 
@@ -936,8 +1065,8 @@ static hipFunction_t segment_kernel_home(cxh_tape_s* t, JitPlan& P, int s, bool 
   home_plan(t, P);
   hipFunction_t& f = soa32 ? P.fwd_home_soa[s] : P.fwd_home[s];
   if (!f)
-    f = jit_function_checked(gen_segment(t, P, s, false, 0, soa32, true), "cxj_fwd",
-                             "use a shorter checkpoint interval or the interpreter engine");
+    f = fast_or_plain([&](bool fast) { return gen_segment(t, P, s, false, 0, soa32, true, fast); }, "cxj_fwd",
+                      "use a shorter checkpoint interval or the interpreter engine");
   return f;
 }
 
@@ -1186,6 +1315,7 @@ static JitPlan& eval_plan(cxh_tape_s* t) {
     for (int g = 0; g < P.n_seg && ok; ++g) {
       if (P.fwd_home[g]) continue;
       hipFunction_t f = jit_function(gen_segment(t, P, g, false, 0, false, true), "cxj_fwd");
+      if (scratch_bytes(f) > 0) f = jit_function(gen_segment(t, P, g, false, 0, false, true, false), "cxj_fwd");
       if (scratch_bytes(f) > 0) {
         ok = false;
       } else {
@@ -1354,16 +1484,17 @@ std::unordered_set<int64_t> step_trig_pairs(const cxh_tape_s* t) {
 
 // Emits `const double v<k> = sin/cos(v<x>)` through sincos (one call per
 // operand, names remembered in trig) and returns true, for SIN / COS when
-// all_trig or the operand is in pairs.
+// all_trig or the operand is in pairs.  wide: the branch-free pair, flagging.
 bool emit_trig(std::string& o, const Instr& e, int64_t k, int64_t x, const std::string& xname, bool all_trig,
                const std::unordered_set<int64_t>& pairs,
-               std::unordered_map<int64_t, std::pair<std::string, std::string>>& trig) {
+               std::unordered_map<int64_t, std::pair<std::string, std::string>>& trig, bool wide) {
   if ((e.op != OP_SIN && e.op != OP_COS) || !(all_trig || pairs.count(x))) return false;
   auto it = trig.find(x);
   if (it == trig.end()) {
     const std::string id = std::to_string(k);
     it = trig.emplace(x, std::make_pair("ts" + id, "tc" + id)).first;
-    o += "  double ts" + id + ", tc" + id + ";\n  CXJ_SINCOS(" + xname + ", ts" + id + ", tc" + id + ");\n";
+    o += "  double ts" + id + ", tc" + id + ";\n  CXJ_SINCOS(" + xname + ", ts" + id + ", tc" + id +
+         (wide ? ", wide);\n" : ");\n");
   }
   o += "  const double v" + std::to_string(k) + " = " + (e.op == OP_SIN ? it->second.first : it->second.second) +
        ";\n";
@@ -2745,15 +2876,13 @@ static MaccPlan macc_plan(const cxh_tape_s* t, int64_t N, int n_accum) {
 // when y is a tape constant the fast division takes; empty otherwise.
 static std::string macc_fast_div(const cxh_tape_s* t, int k, const Instr& e, int64_t x, int64_t y) {
   if (e.op != OP_DIV || t->alg[y].op != OP_CONST || !fast_divisor(t->alg[y].d)) return std::string();
-  const double c = t->alg[y].d;
-  return "  const double v" + std::to_string(k) + " = sxh::sxh_div_c(v" + std::to_string(x) + ", " + lit(c) + ", " +
-         lit(1.0 / c) + ", wide);\n";
+  return "  const double v" + std::to_string(k) + " = " + div_c_call("v" + std::to_string(x), t->alg[y].d) + ";\n";
 }
 
 // Forward step body: state s -> sn, per-step inputs/outputs at column block
 // `step`.  Outputs are written when `outs` is true.  fast: the variant
-// `cxj_step_fwd_f` dividing by constants through sxh_div_c (*ndiv counts
-// them), else `cxj_step_fwd_x` with IEEE division.
+// `cxj_step_fwd_f` dividing by constants through sxh_div_c and taking sin/cos
+// without a branch (*ndiv counts both), else `cxj_step_fwd_x`.
 static std::string gen_macc_step_fwd(const cxh_tape_s* t, const MaccPlan& M, bool fast, int* ndiv = nullptr) {
   std::string o = std::string("__device__ __forceinline__ void cxj_step_fwd") + (fast ? "_f" : "_x") +
                   "(const CxjArgs& A, const long long k, const long long step, const double* s, double* sn, "
@@ -2767,7 +2896,8 @@ static std::string gen_macc_step_fwd(const cxh_tape_s* t, const MaccPlan& M, boo
     const Instr& e = t->alg[kk];
     const int k = static_cast<int>(kk);
     const bool is_trig = e.op == OP_SIN || e.op == OP_COS;
-    if (is_trig && emit_trig(o, e, k, cur[e.i1], "v" + std::to_string(cur[e.i1]), false, pairs, trig)) {
+    if (is_trig && emit_trig(o, e, k, cur[e.i1], "v" + std::to_string(cur[e.i1]), false, pairs, trig, fast)) {
+      if (ndiv) ++*ndiv;
       cur[e.i0] = k;
       continue;
     }
@@ -2827,7 +2957,7 @@ static std::string gen_macc_step_rev(const cxh_tape_s* t, const MaccPlan& M, boo
   for (int k = 0; k < ni; ++k) {
     const Instr& e = t->alg[k];
     const bool is_trig = e.op == OP_SIN || e.op == OP_COS;
-    if (is_trig && emit_trig(o, e, k, cur[e.i1], "v" + std::to_string(cur[e.i1]), true, {}, trig)) {
+    if (is_trig && emit_trig(o, e, k, cur[e.i1], "v" + std::to_string(cur[e.i1]), true, {}, trig, fast)) {
       ox[k] = oy[k] = cur[e.i1];
       cur[e.i0] = k;
       continue;
@@ -2943,8 +3073,8 @@ static std::string gen_macc(const cxh_tape_s* t, const MaccPlan& M, int mode, in
   std::string o = kSxOpsSource;
   o += kPrologue;
   // Modes 0, 2 and 4 (evaluation, checkpointing forward, paired reverse)
-  // divide by tape constants through sxh_div_c in a fast pass and run a loop
-  // again with IEEE division when a lane of the wavefront reported a dividend
+  // divide by tape constants through sxh_div_c and take sin/cos without a
+  // branch in a fast pass, and run a loop again with the exact step when a lane of the wavefront reported a dividend
   // outside its exact range (each pass rewrites every row and output it
   // stores).  The one-launch sweeps (1, 3) divide as IEEE 754 does.
   int nd = 0;
@@ -3097,14 +3227,14 @@ struct CxjTile { long long start; int fun; int pad; };
 // One kernel holding the fused forward + reverse body of every Function of the
 // batch.  Workgroups stride over the tile list (persistent when the grid is
 // smaller than the list); the Function of a tile is wave-uniform.
-static std::string gen_batch(const std::vector<cxh_tape_s*>& tapes) {
+static std::string gen_batch(const std::vector<cxh_tape_s*>& tapes, bool fast = true) {
   std::string o = kSxOpsSource;
   o += kPrologue;
   o += kBatchKernel;
   for (size_t f = 0; f < tapes.size(); ++f) {
     JitPlan& P = plan_for(tapes[f], 0);
     if (P.n_seg != 1) throw std::runtime_error("batch: tape is not a single segment");
-    o += gen_body(tapes[f], P, 0, true, "cxj_f" + std::to_string(f), false);
+    o += gen_whole_body(tapes[f], P, true, "cxj_f" + std::to_string(f), false, false, fast);
   }
   o += "extern \"C\" __global__ void __launch_bounds__(256) cxj_batch(const CxjArgs* __restrict__ args, "
        "const CxjTile* __restrict__ tiles, const long long n_tiles) {\n"
@@ -3386,7 +3516,7 @@ int cxh_batch_create(int32_t n_fun, const cxh_tape* tapes, const int64_t* counts
   }
   b->args.assign(n_fun, CxjArgs{});
   b->bound.assign(n_fun, 0);
-  b->fn = jit_function_checked(gen_batch(b->tapes), "cxj_batch",
+  b->fn = fast_or_plain([&](bool fast) { return gen_batch(b->tapes, fast); }, "cxj_batch",
                                "batch fewer or smaller Functions, or launch them one by one");
   int dev = 0;
   hip_check(hipGetDevice(&dev), "hipGetDevice");

@@ -49,13 +49,23 @@ std::unordered_set<int64_t> step_trig_pairs(const cxh_tape_s* t);
 // `const double v<k> = sin/cos(...)` through one sincos per operand.
 bool emit_trig(std::string& o, const Instr& e, int64_t k, int64_t x, const std::string& xname, bool all_trig,
                const std::unordered_set<int64_t>& pairs,
-               std::unordered_map<int64_t, std::pair<std::string, std::string>>& trig);
+               std::unordered_map<int64_t, std::pair<std::string, std::string>>& trig, bool wide = false);
 
-// Divisions by a tape constant in the loop kernels: whether they go
-// through sxh_div_c (CXH_JIT_FAST_DIV, default on; the same bits either way),
-// and the divisors it takes (finite, 2^-64 <= |c| <= 2^64).
+// Divisions by a tape constant: whether they go through sxh_div_c
+// (CXH_JIT_FAST_DIV, default on; the same bits either way), and the divisors
+// it takes (finite, 2^-64 <= |c| <= 2^64, and no power of two, whose division
+// the compiler turns into an exact product).
 bool fast_div_enabled();
-inline bool fast_divisor(double c) { return std::isfinite(c) && std::fabs(c) >= 0x1p-64 && std::fabs(c) <= 0x1p+64; }
+inline bool fast_divisor(double c) {
+  int e;
+  return std::isfinite(c) && std::fabs(c) >= 0x1p-64 && std::fabs(c) <= 0x1p+64 && std::fabs(std::frexp(c, &e)) != 0.5;
+}
+// Whether x / c = RN(x yh + RN(x yl)) for every x in its range (the two-operation
+// sxh_div_c), decided exactly for the divisor; *yh and *yl are the pair.
+bool div_pair(double c, double* yh, double* yl);
+// `sxh::sxh_div_c(x, c, ..., wide)`: the two-operation form where div_pair
+// accepts c (9275 of 10000 random significands), else the Markstein one.
+std::string div_c_call(const std::string& x, double c);
 
 // hiprtc compile (cached by source) and load; the checked form refuses a
 // kernel that needs scratch, naming the remedy.

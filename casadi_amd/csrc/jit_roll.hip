@@ -375,8 +375,8 @@ struct Emitter {
   // seeds) is recorded here and read from in_[i] instead, the caller issuing
   // the recorded expressions itself (cxj_load_fwd / cxj_load_rev).
   std::vector<std::string>* pre = nullptr;
-  // Divisions by a constant of moderate magnitude through sxh_div_c (the
-  // function declares `bool& wide`); div_c counts them.
+  // Divisions by a constant of moderate magnitude through sxh_div_c and sin/cos
+  // without a branch (the function declares `bool& wide`); div_c counts both.
   bool fast_div = false;
   int64_t div_c = 0;
   char buf[320];
@@ -484,7 +484,10 @@ struct Emitter {
       int64_t kx = 0, ky = 0;
       if (e.op != OP_CONST && e.op != OP_INPUT) operand(k, 1, x, ax, kx);
       if (trig_io && (e.op == OP_SIN || e.op == OP_COS) && trig_row(e, k, kx, x)) continue;
-      if (emit_trig(o, e, k, kx, x, all_trig, pairs, trig)) continue;
+      if (emit_trig(o, e, k, kx, x, all_trig, pairs, trig, fast_div)) {
+        ++div_c;
+        continue;
+      }
       switch (e.op) {
         case OP_CONST:
           o += "  const double v" + ks + " = " + lit(e.d) + ";\n";
@@ -500,8 +503,7 @@ struct Emitter {
           if (op_is_binary(e.op)) operand(k, 2, y, ay, ky);
           else y = x;
           if (fast_div && e.op == OP_DIV && ay.empty() && fast_divisor(t->alg[ky].d)) {
-            const double c = t->alg[ky].d;
-            o += "  const double v" + ks + " = sxh::sxh_div_c(" + x + ", " + lit(c) + ", " + lit(1.0 / c) + ", wide);\n";
+            o += "  const double v" + ks + " = " + div_c_call(x, t->alg[ky].d) + ";\n";
             ++div_c;
             break;
           }
@@ -525,7 +527,9 @@ struct Emitter {
         o += "  const double ts" + id + " = " + load("CXJ_SNAP(st, row0 + " + i + ")") + ";\n  const double tc" + id +
              " = " + load("CXJ_SNAP(st, row0 + " + i + " + 1)") + ";\n";
       } else {
-        o += "  double ts" + id + ", tc" + id + ";\n  CXJ_SINCOS(" + xname + ", ts" + id + ", tc" + id + ");\n";
+        o += "  double ts" + id + ", tc" + id + ";\n  CXJ_SINCOS(" + xname + ", ts" + id + ", tc" +
+             id + (fast_div ? ", wide);\n" : ");\n");
+        ++div_c;
         o += "  if (store_trig) {\n    CXJ_SNAP(st, row0 + " + i + ") = ts" + id + ";\n    CXJ_SNAP(st, row0 + " + i +
              " + 1) = tc" + id + ";\n  }\n";
       }
@@ -647,10 +651,14 @@ std::string gen_functions(const cxh_tape_s* t, const RollPlan& L, bool rev, int6
            ";\n";
     o += "}\n";
   }
-  // The iteration functions: `_x` divides as IEEE 754 does; when the body
-  // divides by constants, `_f` divides through sxh_div_c and reports in
-  // `wide` a dividend outside its exact range (the loops then run again
-  // with `_x`, see gen_roll).
+  // The iteration functions: `_x` divides as IEEE 754 does and branches to
+  // the library's sin/cos past 2^20; when the body divides by constants or
+  // takes a sin or cos, `_f` divides through sxh_div_c, takes them without a
+  // branch and reports in `wide` an operand outside their ranges (the loops
+  // then run again with `_x`, see gen_roll).  One wave per SIMD waits for the
+  // chain of the step: 100 cart-pole steps over 32768 instances, forward and
+  // reverse, 295 us with three corrections per quotient and a branch per pair, 276 with
+  // the two-operation quotient, 268 without the branch.
   *fast = false;
   const bool fast_ok = allow_fast && fast_div_enabled();
   {  // one iteration forward

@@ -195,19 +195,62 @@ SXH_HD double sxh_div_markstein(double x, double y, double yi) {
 // evaluates again with IEEE division.  Short dependent chain (multiply, four
 // FMAs, fixup) and no branch: the kernels that use it are latency-bound
 // single wavefronts whose scheduler needs long straight-line blocks.
+//
+// The second form is two operations, x / c = RN(x yh + RN(x yl)) with yh = 1 / c
+// truncated toward zero and yl = RN(1 / c - yh), which has yh's sign (or c is
+// a power of two), so that zeros, infinities and NaN come out as of x / c
+// (N. Brisebarre, J.-M. Muller, S. K. Raina, "Accelerating correctly rounded
+// floating-point division when the divisor is known in advance", IEEE Trans.
+// Computers 53(8), 2004).  It holds for the divisors div_pair accepts and not
+// for finite nonzero |x| below 2^-900, where x yl or the result may be
+// subnormal: those set `wide`.
 #if defined(__HIPCC_RTC__) || defined(__HIP_DEVICE_COMPILE__)
-SXH_HD double sxh_div_c(double x, double c, double ci, bool& wide) {
-  wide |= static_cast<unsigned>(__builtin_amdgcn_frexp_exp(x) + 899) > 1800u;
+// Straight-line bodies collect their flags in a lane mask that the compiler
+// cannot compute later: left to itself it moves the comparisons to the end of
+// the body and keeps every operand live until there (90 registers in place of 60
+// in the map of a cart-pole step).  Loop bodies are faster with a plain flag.
+struct WaveFlag {
+  unsigned long long m = 0;
+  SXH_HD bool any() const { return m != 0; }
+};
+SXH_HD void sxh_flag(bool b, bool& wide) { wide |= b; }
+SXH_HD void sxh_flag(bool b, WaveFlag& wide) {
+  unsigned long long m = __builtin_amdgcn_ballot_w64(b);
+  asm volatile("" : "+s"(m));
+  wide.m |= m;
+}
+template <class W>
+SXH_HD double sxh_div_c(double x, double, double yh, double yl, W& wide) {
+  sxh_flag(__builtin_amdgcn_frexp_exp(x) < -899, wide);
+  return fma(x, yh, x * yl);
+}
+template <class W>
+SXH_HD double sxh_div_c(double x, double c, double ci, W& wide) {
+  sxh_flag(static_cast<unsigned>(__builtin_amdgcn_frexp_exp(x) + 899) > 1800u, wide);
   return __builtin_amdgcn_div_fixup(sxh_div_markstein(fabs(x), fabs(c), fabs(ci)), c, x);
 }
 #else
 // The same on the host (the kernels' host emulation): frexp's exponent is 0
 // for zero, infinity and NaN as v_frexp_exp_i32_f64 gives it, and the fixup
 // follows v_div_fixup_f64 for a finite nonzero divisor c and a quotient q >= 0.
-SXH_HD double sxh_div_c(double x, double c, double ci, bool& wide) {
+struct WaveFlag {
+  bool m = false;
+  bool any() const { return m; }
+};
+inline void sxh_flag(bool b, bool& wide) { wide |= b; }
+inline void sxh_flag(bool b, WaveFlag& wide) { wide.m |= b; }
+template <class W>
+SXH_HD double sxh_div_c(double x, double, double yh, double yl, W& wide) {
   int e = 0;
   if (std::isfinite(x)) std::frexp(x, &e);
-  wide |= static_cast<unsigned>(e + 899) > 1800u;
+  wide |= e < -899;
+  return std::fma(x, yh, x * yl);
+}
+template <class W>
+SXH_HD double sxh_div_c(double x, double c, double ci, W& wide) {
+  int e = 0;
+  if (std::isfinite(x)) std::frexp(x, &e);
+  sxh_flag(static_cast<unsigned>(e + 899) > 1800u, wide);
   const double q = sxh_div_markstein(std::fabs(x), std::fabs(c), std::fabs(ci));
   const bool neg = std::signbit(x) != std::signbit(c);
   if (std::isnan(x)) return x + x;
@@ -235,7 +278,7 @@ SXH_HD double sxh_div_c(double x, double c, double ci, bool& wide) {
 // arithmetic: at most 0.682, mean 0.2515; the device library's sincos, which
 // it replaces, at most 0.768, mean 0.2541.  About as many instructions as the
 // library's (45 against 48 per pair), but a shorter dependent chain, which is
-// what kernels with one wave per SIMD wait for: a 100-step pendulum rollout's
+// what kernels with one wave per SIMD wait for: a 100-step cart-pole rollout's
 // gradient over 32768 instances 319 -> 295 us, the Hessian of 20 stages over
 // 16384 249 -> 238 us, the issue-bound map over 8388608 162 -> 156 us.
 SXH_HD void sxh_sincos_reduced(double x, double* s, double* c) {
@@ -273,6 +316,17 @@ SXH_HD void sxh_sincos(double x, double* s, double* c) {
 #else
   *s = sin(x);
   *c = cos(x);
+#endif
+}
+// The pair without a branch: a finite |x| past 2^20 (and an infinity) sets
+// `wide`, and the caller then evaluates again with sxh_sincos.  NaN in, NaN out.
+template <class W>
+SXH_HD void sxh_sincos(double x, double* s, double* c, W& wide) {
+#if defined(__HIPCC_RTC__) || defined(__HIP_DEVICE_COMPILE__)
+  sxh_sincos_reduced(x, s, c);
+  sxh_flag(fabs(x) > 0x1p20, wide);
+#else
+  sxh_sincos(x, s, c);
 #endif
 }
 SXH_HD double sxh_sin(double x) {
