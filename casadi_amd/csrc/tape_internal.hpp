@@ -77,9 +77,9 @@ struct cxh_tape_s {
   int64_t ws = 1;
   std::vector<int64_t> nnz_in, nnz_out;
   std::vector<int2> unused_in;
-  sxh::DeviceBuffer d_tape, d_unused;  // uploaded at first interpreter launch
-  sxh::DeviceBuffer d_live;            // adjoint_live bits, uploaded at the first interpreter adjoint
-  bool uploaded = false;
+  sxh::DeviceBuffer d_tape;                   // uploaded at the first tangent or sparsity launch
+  sxh::DeviceBuffer d_code, d_imm, d_unused;  // uploaded at the first interpreter evaluation or adjoint
+  bool uploaded = false, coded = false;
   sxh::DeviceBuffer scratch, trail, ckpt;
   sxh::DeviceBuffer red, partial;  // summed blocks of a reduced map (mapsum.hip)
   sxh::DeviceBuffer spw;           // work words of a sparsity sweep too large for LDS (sparsity_kernels.hip)
