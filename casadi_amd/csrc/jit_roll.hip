@@ -657,7 +657,7 @@ std::string gen_functions(const cxh_tape_s* t, const RollPlan& L, bool rev, int6
   // branch and reports in `wide` an operand outside their ranges (the loops
   // then run again with `_x`, see gen_roll).  One wave per SIMD waits for the
   // chain of the step: 100 cart-pole steps over 32768 instances, forward and
-  // reverse, 295 us with three corrections per quotient and a branch per pair, 276 with
+  // reverse, 295 us with two corrections per quotient and a branch per pair, 276 with
   // the two-operation quotient, 268 without the branch.
   *fast = false;
   const bool fast_ok = allow_fast && fast_div_enabled();
