@@ -68,6 +68,7 @@ cxh_tape_jit_fallback = _fn("cxh_tape_jit_fallback", I32, P, C.c_char_p, I64)
 cxh_tape_tune = _fn("cxh_tape_tune", I32, P, I64, PP, PP, I32, I64, I32, P, C.POINTER(I32), C.POINTER(C.c_double))
 cxh_map_eval = _fn("cxh_map_eval", I32, P, I64, PP, PP, I32, I64, P)
 cxh_map_eval_host = _fn("cxh_map_eval_host", I32, P, I64, PP, PP)
+cxh_map_eval_host_soa = _fn("cxh_map_eval_host_soa", I32, P, I64, PP, PP)
 cxh_map_fwd_adj = _fn("cxh_map_fwd_adj", I32, P, I64, PP, PP, PP, PP, I32, I64, I64, P)
 cxh_tape_regularity_check = _fn("cxh_tape_regularity_check", I32, P, I32, P, I64)
 cxh_tape_io = _fn("cxh_tape_io", I32, P, C.POINTER(I32), C.POINTER(I32), PI64, PI64)

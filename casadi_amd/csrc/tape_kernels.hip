@@ -1199,35 +1199,53 @@ int map_eval_io(cxh_tape t, int64_t n, const IOTable& d_arg, const IOTable& d_re
 
 extern "C" {
 
+// One device allocation for all blocks, each starting on 256 bytes.
+static int map_eval_host(cxh_tape t, int64_t n, const double* const* arg, double* const* res, int32_t layout) {
+  const size_t ni = t->nnz_in.size(), no = t->nnz_out.size();
+  auto bytes = [&](int64_t nnz) { return static_cast<size_t>(n) * nnz * sizeof(double); };
+  auto room = [&](int64_t nnz) { return (bytes(nnz) + 255) / 256 * 256; };
+  size_t total = 0;
+  for (size_t i = 0; i < ni; ++i)
+    if (arg[i]) total += room(t->nnz_in[i]);
+  for (size_t i = 0; i < no; ++i)
+    if (res[i]) total += room(t->nnz_out[i]);
+  DeviceBuffer d;
+  if (total) d.reserve(total);
+  char* at = d.as<char>();
+  std::vector<const double*> pa(ni, nullptr);
+  std::vector<double*> pr(no, nullptr);
+  for (size_t i = 0; i < ni; ++i)
+    if (arg[i] && t->nnz_in[i] > 0) {
+      hip_check(hipMemcpy(at, arg[i], bytes(t->nnz_in[i]), hipMemcpyHostToDevice), "hipMemcpy H2D");
+      pa[i] = reinterpret_cast<const double*>(at);
+      at += room(t->nnz_in[i]);
+    }
+  for (size_t i = 0; i < no; ++i)
+    if (res[i] && t->nnz_out[i] > 0) {
+      pr[i] = reinterpret_cast<double*>(at);
+      at += room(t->nnz_out[i]);
+    }
+  int rc = cxh_map_eval(t, n, pa.data(), pr.data(), layout, n, nullptr);
+  if (rc) return rc;
+  for (size_t i = 0; i < no; ++i)
+    if (pr[i]) hip_check(hipMemcpy(res[i], pr[i], bytes(t->nnz_out[i]), hipMemcpyDeviceToHost), "hipMemcpy D2H");
+  hip_check(hipDeviceSynchronize(), "hipDeviceSynchronize");
+  return 0;
+}
+
 int cxh_map_eval_host(cxh_tape t, int64_t n, const double* const* arg, double* const* res) {
   CXH_TRY
   if (!t) return cxh_fail("null tape");
   if (n <= 0) return 0;
-  const size_t ni = t->nnz_in.size(), no = t->nnz_out.size();
-  std::vector<DeviceBuffer> din(ni), dout(no);
-  std::vector<const double*> pa(ni, nullptr);
-  std::vector<double*> pr(no, nullptr);
-  for (size_t i = 0; i < ni; ++i) {
-    if (arg[i] && t->nnz_in[i] > 0) {
-      din[i].upload(arg[i], static_cast<size_t>(n) * t->nnz_in[i] * sizeof(double));
-      pa[i] = din[i].as<double>();
-    }
-  }
-  for (size_t i = 0; i < no; ++i) {
-    if (res[i] && t->nnz_out[i] > 0) {
-      dout[i].reserve(static_cast<size_t>(n) * t->nnz_out[i] * sizeof(double));
-      pr[i] = dout[i].as<double>();
-    }
-  }
-  int rc = cxh_map_eval(t, n, pa.data(), pr.data(), CXH_AOS, n, nullptr);
-  if (rc) return rc;
-  for (size_t i = 0; i < no; ++i)
-    if (pr[i])
-      hip_check(hipMemcpy(res[i], pr[i], static_cast<size_t>(n) * t->nnz_out[i] * sizeof(double),
-                          hipMemcpyDeviceToHost),
-                "hipMemcpy D2H");
-  hip_check(hipDeviceSynchronize(), "hipDeviceSynchronize");
-  return 0;
+  return map_eval_host(t, n, arg, res, CXH_AOS);
+  CXH_CATCH
+}
+
+int cxh_map_eval_host_soa(cxh_tape t, int64_t n, const double* const* arg, double* const* res) {
+  CXH_TRY
+  if (!t) return cxh_fail("null tape");
+  if (n <= 0) return 0;
+  return map_eval_host(t, n, arg, res, CXH_SOA);
   CXH_CATCH
 }
 

@@ -323,6 +323,19 @@ class HipTape:
         L.check(L.cxh_map_eval_host(self._h, n, pa, pr), "cxh_map_eval_host")
         return res
 
+    def eval_host_soa(self, args, n):
+        """Host arrays of one row per nonzero and one column per instance
+        (None: zeros): copied to the device as they are."""
+        arg = [np.ascontiguousarray(a, dtype=float) if a is not None else None for a in args]
+        for a, k in zip(arg, self.nnz_in):
+            if a is not None and a.shape != (k, n):
+                raise ValueError(f"host block has shape {a.shape}, expected {(k, n)}")
+        res = [np.empty((k, n)) for k in self.nnz_out]
+        pa = L.ptr_array([a.ctypes.data if a is not None and a.size else None for a in arg])
+        pr = L.ptr_array([r.ctypes.data if r.size else None for r in res])
+        L.check(L.cxh_map_eval_host_soa(self._h, n, pa, pr), "cxh_map_eval_host_soa")
+        return res
+
     # -- adjoint ---------------------------------------------------------------
     def fwd_adj(self, args, seeds, n=None, checkpoint_every=0, res=True, stream=None):
         """Primal outputs and adj_in = J^T seeds for every instance, one launch."""

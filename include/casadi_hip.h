@@ -250,6 +250,9 @@ int cxh_map_eval(cxh_tape t, int64_t n, const double* const* arg, double* const*
 /* Same as cxh_map_eval on HOST arrays in CasADi's AoS Map layout
  * (the drop-in for Map::eval's arg/res); synchronous.                       */
 int cxh_map_eval_host(cxh_tape t, int64_t n, const double* const* arg, double* const* res);
+/* The same on host blocks [nonzero][instance]: nonzero j of instance k of
+ * block i at arg[i][j*n + k]. */
+int cxh_map_eval_host_soa(cxh_tape t, int64_t n, const double* const* arg, double* const* res);
 
 /* Fused forward + adjoint sweep (one launch): primal outputs res and the
  * gradient adj_in = (d out / d in)^T adj_out for every instance.
