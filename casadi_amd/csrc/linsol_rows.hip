@@ -138,7 +138,10 @@ __device__ __forceinline__ double cxr_fetch(const CxrArgs& A, int e, long long i
   CXR_FROM(3, A.d, i * 8, A.ld)
   return *(const double*)(p + (unsigned long long)k * (unsigned long long)s);
 }
-// a pivot's block
+// a pivot's block.  Every lane reads, a lane above those of the mask one value
+// past them: the next block's first, which must be there.  A block of one
+// value is read by all lanes alike (the last one is: nothing follows it).
+#define CXR_KEPT1(off) *(const double*)(A.w + (off) * 8 + w_at)
 #define CXR_KEPT(off, m) *(const double*)(A.w + (off) * 8 + (CXR_RANK(m) * 8u + w_at))
 #define CXR_KEEP_BLOCK(off, m, v) do { if (CXR_IN(m)) *(double*)(A.w + (off) * 8 + (CXR_RANK(m) * 8u + w_at)) = (v); } while (0)
 // scattered stores of the factor's rows, instance i
@@ -502,8 +505,9 @@ bool rows_ldl_source(int n, const std::vector<int>& a_colind, const std::vector<
     E.out += "  CXR_SYNC();\n";
     for (int j = 0; j < kBack; ++j) E.out += "  vd k" + S(j) + " = 0.0;\n";
     auto kept = [&](int r) {
-      return r >= 0 ? "  k" + S(r % kBack) + " = CXR_KEPT(" + S(block[r]) + ", " + hexmask(mem[r] | 1u << lane[r]) + ");\n"
-                    : std::string();
+      if (r < 0) return std::string();
+      const std::string v = "  k" + S(r % kBack) + " = ", at = S(block[r]);
+      return v + (mem[r] ? "CXR_KEPT(" + at + ", " + hexmask(mem[r] | 1u << lane[r]) + ");\n" : "CXR_KEPT1(" + at + ");\n");
     };
     for (int j = 1; j <= kBack; ++j) E.body += kept(n - j);
     for (int r = n - 1; r >= 0; --r) {
@@ -717,7 +721,7 @@ bool rows_qr_source(int ncol, int nrow, const std::vector<int>& a_colind, const 
   if (solve) {  // back substitution with R: x(r) in column r's lane
     E.out += "  CXR_SYNC();\n";
     for (int j = 0; j < kBack; ++j) E.out += "  vd k" + S(j) + " = 0.0;\n";
-    auto kept = [&](int r) {
+    auto kept = [&](int r) {  // lane 15 is in every mask: no lane reads past a block
       return r >= 0 ? "  k" + S(r % kBack) + " = CXR_KEPT(" + S(block[r]) + ", " + hexmask(mems[r]) + ");\n" : std::string();
     };
     for (int j = 1; j <= kBack; ++j) E.body += kept(ncol - j);

@@ -102,11 +102,13 @@ static vd rows_ring(const double* ring, int start, unsigned m) {
     if (m >> l & 1u) r.v[l] = ring[start + rows_rank(m, l)];
   return r;
 }
+// every lane of the wavefront reads, the lanes outside the mask a value that
+// nothing uses
 static vd rows_kept(const char* w, unsigned m) {
   vd r(NAN);
   for (int l = 0; l < 16; ++l) {
     const char* p = w + rows_rank(m, l) * 8;
-    if ((m >> l & 1u) && rows_emu::inside(p)) r.v[l] = *reinterpret_cast<const double*>(p);
+    if (rows_emu::inside(p) && (m >> l & 1u)) r.v[l] = *reinterpret_cast<const double*>(p);
   }
   return r;
 }
@@ -145,6 +147,7 @@ static vd rows_sel(unsigned m, const vd& a, const vd& b) {
 #define CXR_FETCH(e_) rows_batch(A, e_, i)
 #define CXR_LAND(b, x) do { for (int l = 0; l < 16; ++l) ring[((b) % 8) * 16 + l] = (x).v[l]; } while (0)
 #define CXR_RING(start, m) rows_ring(ring, start, static_cast<unsigned>(m))
+#define CXR_KEPT1(off) (rows_emu::inside(A.w + i * A.w_t + (off) * 8) ? vd(*(const double*)(A.w + i * A.w_t + (off) * 8)) : vd(NAN))
 #define CXR_KEPT(off, m) rows_kept(A.w + i * A.w_t + (off) * 8, static_cast<unsigned>(m))
 #define CXR_KEEP_BLOCK(off, m, v) rows_keep(A.w + i * A.w_t + (off) * 8, static_cast<unsigned>(m), v)
 template <class Args>
