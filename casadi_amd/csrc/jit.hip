@@ -2409,6 +2409,7 @@ int jit_map_jac(cxh_jac_s* j, int64_t n, const IOTable& arg, const IOTable& res,
 // does not split).
 std::string jit_parts_source(cxh_jac_s* j, bool soa32, int* n_units, int* spill_rows, std::vector<int>* rows) {
   *n_units = *spill_rows = 0;
+  if (!parts_enabled()) return "";
   JitParts& P = parts_of(j);
   if (P.cls.empty()) return "";
   *rows = P.rows;

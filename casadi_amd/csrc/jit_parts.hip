@@ -40,7 +40,7 @@ namespace sxh {
 
 namespace {
 
-constexpr int64_t kMaxPart = 4096;  // instructions of one part's program: one kernel, no segments
+constexpr int64_t kMaxPart = 4096;  // instructions of one part's program, its inputs and constants included: one kernel
 constexpr int64_t kSmall = 512;    // classes with fewer instructions in all run together as one part
 
 struct Part {
@@ -241,7 +241,7 @@ std::vector<std::unique_ptr<PartClass>> find_parts(const cxh_jac_s* j, std::vect
     longest = std::max(longest, static_cast<int64_t>(parts[g[0]].instr.size()));
     ops += work(g);
   }
-  if (longest * 2 > ops || longest > kMaxPart || groups.size() > 16) return out;
+  if (longest * 2 > ops || longest > kMaxPart || groups.size() > 16) return out;  // and the localised part, below
   for (const auto& g : groups) {
     const int64_t first = static_cast<int64_t>(rows.size());
     std::unique_ptr<PartClass> C;
@@ -250,9 +250,14 @@ std::vector<std::unique_ptr<PartClass>> find_parts(const cxh_jac_s* j, std::vect
       auto L = localise(j, parts[p].instr, d1, d2, rows, s);
       if (!C) C = std::move(L);
     }
+    if (static_cast<int64_t>(C->tape.alg.size()) > kMaxPart) {
+      rows.clear();
+      return {};
+    }
     C->count = static_cast<int>(g.size());
     C->first_row = first;
     C->jac.tape = &C->tape;
+    C->jac.seg_len = kMaxPart;  // one kernel
     out.push_back(std::move(C));
   }
   return out;

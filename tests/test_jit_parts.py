@@ -115,6 +115,29 @@ def test_tapes_that_do_not_split():
     assert HipJacobian(ca.Function("chain", [x], [ca.vertcat(*[chain * x[i] for i in range(8)])]), engine="jit").parts_source() is None
 
 
+def _chains(ops, n_part=3, n_param=40):
+    """n_part chains of `ops` operations on a differentiated input and n_param parameters each."""
+    import casadi_amd as ca
+    x, p = ca.SX.sym("x", n_part), ca.SX.sym("p", n_part * n_param)
+    out = []
+    for k in range(n_part):
+        c = x[k]
+        for i in range(ops):
+            c = ca.sin(c) if i % 2 == 0 else c * p[n_param * k + (i // 2) % n_param]
+        out.append(c)
+    return ca.Function("chains", [x, p], [ca.vertcat(*out)])
+
+
+def test_longest_part_counts_its_inputs():
+    """A part's program loads 41 inputs and stores one output beside its
+    operations: 4096 instructions are one kernel, 4097 leave the whole-tape
+    kernels to serve the call."""
+    from casadi_amd.hip import HipJacobian
+    plan = lambda ops: HipJacobian(_chains(ops), first_block=True, engine="jit")
+    assert plan(4096 - 42).parts_source() is not None
+    assert plan(4097 - 42).parts_source() is None
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind,n", [("ocp2", 1), ("ocp4", 65), ("ocp4", 1001), ("regular", 63), ("irregular", 200)])
 def test_parts_keep_the_bits(cuda, monkeypatch, kind, n):
