@@ -1551,7 +1551,9 @@ static int jac_dir_group(int ndir, int64_t n) {
 }
 
 static JitJac& jac_plan(cxh_jac_s* j, int64_t n) {
-  const int want = j->ndir == 0 ? 1 : j->dir_group > 0 ? std::min(j->dir_group, std::max(j->ndir, 1)) : std::min(std::max(j->ndir, 1), std::min(jac_dir_group(j->ndir, n), 64));
+  // at most 64: a group's directions are bits of one word
+  const int want =
+      j->ndir == 0 ? 1 : std::min({j->ndir, 64, j->dir_group > 0 ? j->dir_group : jac_dir_group(j->ndir, n)});
   if (j->jit && j->jit->group == want) return *j->jit;
   const cxh_tape_s* t = j->tape;
   auto J = std::make_shared<JitJac>();

@@ -138,6 +138,22 @@ def test_longest_part_counts_its_inputs():
     assert plan(4097 - 42).parts_source() is None
 
 
+def test_direction_groups_hold_at_most_64(monkeypatch):
+    """A group's directions are bits of a 64-bit mask, whatever the setting asks for."""
+    import casadi_amd as ca
+    from casadi_amd.hip import HipJacobian
+    monkeypatch.setenv("CXH_JIT_DIRGROUP", "80")
+    x = ca.SX.sym("x", 3 * 80)
+    out = []
+    for k in range(3):
+        s = sum(ca.sin(x[80 * k + i]) * x[80 * k + (i + 1) % 80] for i in range(80))
+        out += [s * x[80 * k + i % 80] for i in range(90)]
+    h = HipJacobian(ca.Function("wide", [x], [ca.vertcat(*out)]), engine="jit")
+    src, _, units, _ = h.parts_source()
+    groups = len(re.findall(r"case \d+: cxj_body_c\d+_g\d+", src))
+    assert h.plan["ndir"] == 80 and groups == 2 and units == 3 * groups
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind,n", [("ocp2", 1), ("ocp4", 65), ("ocp4", 1001), ("regular", 63), ("irregular", 200)])
 def test_parts_keep_the_bits(cuda, monkeypatch, kind, n):
