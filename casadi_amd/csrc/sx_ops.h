@@ -243,7 +243,7 @@ template <class W>
 SXH_HD double sxh_div_c(double x, double, double yh, double yl, W& wide) {
   int e = 0;
   if (std::isfinite(x)) std::frexp(x, &e);
-  wide |= e < -899;
+  sxh_flag(e < -899, wide);
   return std::fma(x, yh, x * yl);
 }
 template <class W>
@@ -327,6 +327,7 @@ SXH_HD void sxh_sincos(double x, double* s, double* c, W& wide) {
   sxh_flag(fabs(x) > 0x1p20, wide);
 #else
   sxh_sincos(x, s, c);
+  sxh_flag(fabs(x) > 0x1p20, wide);
 #endif
 }
 SXH_HD double sxh_sin(double x) {
