@@ -268,15 +268,18 @@ SXH_HD double sxh_div_c(double x, double c, double ci, W& wide) {
 // 53, 33 and 53 bits.  x - k P1 is exact (a multiple of 2^-53 below 1), and so
 // is what its difference r to k P2 (a multiple of 2^-87, |k| < 2^20) rounds
 // off, so the reduced argument is r + rl with rl that remainder and the P3
-// term.  Then
-// minimax polynomials on |r| <= pi/4 (Remez; relative error 2^-57.9 for sin,
-// 2^-63.9 for cos), the leading terms added last with their corrections for
-// rl, for the rounding of 1 - r^2/2 and for that of r^2.
+// term.  Then minimax polynomials on |r| <= pi/4 (Remez; with their rounded
+// coefficients within 2^-56.5 of sin and 2^-59.3 of cos, relatively), the leading
+// terms added last with their corrections for rl, for the rounding of 1 - r^2/2
+// and for that of r^2: the arrangement of fdlibm's __kernel_sin and __kernel_cos
+// (Sun Microsystems, 1993).
 //
-// Error, in ulps over 200 000 arguments in each of +-0.8, +-10 (half of them
-// next to multiples of pi/2), +-1000 and +-2^20, against 113-bit
-// arithmetic: at most 0.682, mean 0.2515; the device library's sincos, which
-// it replaces, at most 0.768, mean 0.2541.  About as many instructions as the
+// Error: the sine at |r| = pi/4 is the worst, 0.5 ulp for the last addition, 0.11
+// for r^2 and r^3 rounded in r^3 / 6, 0.07 for the roundings of what is
+// subtracted and 0.06 for the polynomial, 0.74 in all.  Over 100 million
+// arguments in each of +-0.8, +-1, +-10, +-1000 and +-2^20, against a 64-bit
+// significand: at most 0.726, mean 0.2509.  The device library's sincos, which
+// it replaces, over 800 000 arguments: at most 0.768, mean 0.2541.  About as many instructions as the
 // library's (45 against 48 per pair), but a shorter dependent chain, which is
 // what kernels with one wave per SIMD wait for: a 100-step cart-pole rollout's
 // gradient over 32768 instances 319 -> 295 us, the Hessian of 20 stages over

@@ -2,9 +2,12 @@
 host (the same IEEE operations) against 64-bit-significand arithmetic, on the
 GPU against the host's bits through both engines.
 
-Bound: |r| <= pi/4, so each result is a leading term (r or 1 - r^2/2, at most
-half an ulp off after the last addition) plus corrections below a quarter of
-it whose own roundings add up to less than a fifth of an ulp."""
+Bound, at |r| = pi/4, where it is largest (the sine there lies in [0.5, 1), in
+units of its ulp, 2^-53): half for the last subtraction; r^2 is rounded by half
+and r^3 by a quarter of a unit, which reach r^3 / 6 as 0.065 and 0.042; the
+subtracted r^3 / 6 - ... lies below 1/8 and is rounded by 1/16, its inner terms
+add 0.01; the polynomial with rounded coefficients is within 2^-56.5 of the
+sine, 0.06.  0.74 in all."""
 import ctypes as C
 import os
 import subprocess
@@ -55,7 +58,7 @@ def test_reduced_sincos_error(reduced):
     for got, ref in ((s, np.sin(xl)), (c, np.cos(xl))):
         ulp = np.spacing(np.abs(ref.astype(np.float64))).astype(np.longdouble)
         err = np.abs(got.astype(np.longdouble) - ref) / ulp
-        assert err.max() <= 0.7 and err.mean() <= 0.26
+        assert err.max() <= 0.75 and err.mean() <= 0.26
 
 
 def test_reduced_sincos_zeros(reduced):
