@@ -29,6 +29,7 @@
 #include <cstring>
 #include <map>
 #include <numeric>
+#include <set>
 #include <string>
 #include <utility>
 #include <vector>
@@ -183,6 +184,7 @@ std::vector<std::unique_ptr<PartClass>> find_parts(const cxh_jac_s* j, std::vect
   auto meets = [&](int64_t k, int64_t u) {
     if (u >= 0 && t->alg[u].op != OP_CONST && t->alg[u].op != OP_INPUT) up[root(up, u)] = root(up, k);
   };
+  std::set<std::pair<int, int>> written;
   for (int64_t k = 0; k < n; ++k) {
     const Instr& e = t->alg[k];
     if (e.op == OP_CONST || e.op == OP_INPUT) {
@@ -190,7 +192,10 @@ std::vector<std::unique_ptr<PartClass>> find_parts(const cxh_jac_s* j, std::vect
       continue;
     }
     meets(k, d1[k] = cur[e.i1]);
-    if (e.op == OP_OUTPUT) continue;
+    if (e.op == OP_OUTPUT) {
+      if (!written.insert({e.i0, e.i2}).second) return out;  // the last write counts, and parts have no order
+      continue;
+    }
     if (op_is_binary(e.op)) meets(k, d2[k] = cur[e.i2]);
     cur[e.i0] = k;
   }

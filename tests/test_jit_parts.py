@@ -154,6 +154,20 @@ def test_direction_groups_hold_at_most_64(monkeypatch):
     assert h.plan["ndir"] == 80 and groups == 2 and units == 3 * groups
 
 
+def test_an_output_written_twice_keeps_the_order():
+    """The last of several writes to one output nonzero counts; parts run in no
+    order, so such a tape stays whole."""
+    from casadi_amd.hip import HipJacobian, HipTape
+    from casadi_amd.ops import OP
+    f = _chains(600)
+    prog = np.array(f.instructions())
+    tape = lambda p: HipTape.nested(p, int(p["i0"].max()) + 1, [3, 120], [3], [], engine="jit")
+    assert HipJacobian(f, tape=tape(prog), first_block=True).parts_source() is not None
+    outs = np.flatnonzero(prog["op"] == OP.OUTPUT)
+    prog["i2"][outs[-1]] = prog["i2"][outs[0]]
+    assert HipJacobian(f, tape=tape(prog), first_block=True).parts_source() is None
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind,n", [("ocp2", 1), ("ocp4", 65), ("ocp4", 1001), ("regular", 63), ("irregular", 200)])
 def test_parts_keep_the_bits(cuda, monkeypatch, kind, n):
