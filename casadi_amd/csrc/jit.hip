@@ -111,6 +111,7 @@ struct CxjArgs {
 #else
 #define CXJ_SINCOS(x_, s_, c_, ...) sxh::sxh_sincos(x_, &s_, &c_, ##__VA_ARGS__)
 #endif
+#define CXJ_SINCOS_COLD(x_, s_, c_) CXJ_SINCOS(x_, s_, c_)
 )CXJ";
 
 // Sites of sin/cos pairs above which a program calls one out-of-line copy
@@ -125,7 +126,7 @@ static int trig_call_sites() {
 std::string finish_source(std::string o) {
   const int lim = trig_call_sites();
   if (lim < 0) return o;
-  int64_t sites = 0;  // "  CXJ_SINCOS(" starts an emitted line; the definitions have one space
+  int64_t sites = 0;  // "  CXJ_SINCOS(" starts an emitted line; the definitions have one space, cold sites another name
   for (size_t p = o.find("  CXJ_SINCOS("); p != std::string::npos; p = o.find("  CXJ_SINCOS(", p + 1)) ++sites;
   return sites > lim ? "#define CXJ_TRIG_CALLS\n" + o : o;
 }
@@ -482,13 +483,15 @@ static std::string adj_name(int64_t c, int64_t ws) {
 // sensitivity back to the end (an output may be written over an input), and
 // evaluate again with `<name>_x`, which divides as IEEE 754 does and calls the
 // library's sincos past 2^20, when a lane of the wavefront reported an operand
-// outside their ranges; *div counts the divisions and pairs.  The body is bound
+// outside their ranges; *div counts the divisions and pairs.  cold: that exact
+// body, whose sin/cos sites do not count towards trig_call_sites().  The body is bound
 // by the instructions it issues (with few instances, by its chain), and an IEEE division is
 // eleven of them against four: the map of a cart-pole RK4 step (12
 // divisions, 4 pairs) over 8388608 instances 155.7 -> 130 us, the summed map's
 // gradient over 1048576 44.4 -> 41.7, a mixed batch of 77000 12.3 -> 11.6.
 static std::string gen_body(const cxh_tape_s* t, const JitPlan& P, int s, bool rev, const std::string& name,
-                            bool sub_blocks = true, int phase = 0, bool home = false, int* div = nullptr) {
+                            bool sub_blocks = true, int phase = 0, bool home = false, int* div = nullptr,
+                            bool cold = false) {
   const int t0 = P.t0[s], t1 = P.t0[s + 1];
   const int len = t1 - t0;
   const int64_t ws = t->ws;
@@ -625,7 +628,7 @@ static std::string gen_body(const cxh_tape_s* t, const JitPlan& P, int s, bool r
             o += "  const double ts" + id + " = CXJ_SNAP(" + trig_ptr + ", " + std::to_string(r) + "), tc" + id +
                  " = CXJ_SNAP(" + trig_ptr + ", " + std::to_string(r + 1) + ");\n";
           } else {
-            o += "  double ts" + id + ", tc" + id + ";\n  CXJ_SINCOS(" + V(x) + ", ts" + id + ", tc" + id +
+            o += "  double ts" + id + ", tc" + id + (cold ? ";\n  CXJ_SINCOS_COLD(" : ";\n  CXJ_SINCOS(") + V(x) + ", ts" + id + ", tc" + id +
                  (div ? ", wide);\n" : ");\n");
             if (div) ++*div;
           }
@@ -891,8 +894,7 @@ static std::string gen_body(const cxh_tape_s* t, const JitPlan& P, int s, bool r
 constexpr int64_t kHeldEval = 32, kHeldReverse = 16;
 
 // gen_body of a tape that is one segment swept in one piece, with its divisions
-// by constants and sin/cos flagged (see gen_body) where that pays: the exact body
-// behind it is cold, so its sin/cos sites do not count towards trig_call_sites().
+// by constants and sin/cos flagged (see gen_body) where that pays.
 static std::string gen_whole_body(const cxh_tape_s* t, const JitPlan& P, bool rev, const std::string& name, bool sub_blocks,
                                   bool home, bool fast) {
   int64_t held = 0;
@@ -903,10 +905,7 @@ static std::string gen_whole_body(const cxh_tape_s* t, const JitPlan& P, bool re
     int nd = 0;
     const std::string f = gen_body(t, P, 0, rev, name, sub_blocks, 0, home, &nd);
     if (nd > 0) {
-      std::string x = gen_body(t, P, 0, rev, name + "_x", sub_blocks, 0, home);
-      const std::string site = "  CXJ_SINCOS(";
-      for (size_t p = x.find(site); p != std::string::npos; p = x.find(site, p)) x.replace(p, site.size(), "\n CXJ_SINCOS(");
-      return x + f;
+      return gen_body(t, P, 0, rev, name + "_x", sub_blocks, 0, home, nullptr, true) + f;
     }
   }
   return gen_body(t, P, 0, rev, name, sub_blocks, 0, home);
