@@ -2344,18 +2344,8 @@ static bool parts_map_jac(cxh_jac_s* j, int64_t n, CxjArgs A, hipStream_t s) {
   return true;
 }
 
-int jit_map_jac(cxh_jac_s* j, int64_t n, const IOTable& arg, const IOTable& res, double* jac, int64_t jac_s_nz,
-                int64_t jac_s_inst, hipStream_t s) {
-  if (j->ndir > 0 && (!j->parts || !j->parts->cls.empty())) {
-    CxjArgs A{};
-    A.arg = arg;
-    A.res = res;
-    A.asens.a[0] = {jac, jac_s_nz, jac_s_inst};
-    A.n = n;
-    A.lds = round_up(n, 64);
-    if (parts_map_jac(j, n, A, s)) return 0;
-  }
-  JitJac& J = jac_plan(j, n);
+// The kernels of a plan, compiled.
+static void jac_build(cxh_jac_s* j, JitJac& J) {
   for (int sg = 0; sg < J.n_seg; ++sg) {
     hipFunction_t& f = J.fn[sg];
     // the budget counts values, not the compiler's temporaries: where the
@@ -2369,6 +2359,21 @@ int jit_map_jac(cxh_jac_s* j, int64_t n, const IOTable& arg, const IOTable& res,
       J.spill_rows = std::max<int64_t>(J.spill_rows, ns);
     }
   }
+}
+
+int jit_map_jac(cxh_jac_s* j, int64_t n, const IOTable& arg, const IOTable& res, double* jac, int64_t jac_s_nz,
+                int64_t jac_s_inst, hipStream_t s) {
+  if (j->ndir > 0 && (!j->parts || !j->parts->cls.empty())) {
+    CxjArgs A{};
+    A.arg = arg;
+    A.res = res;
+    A.asens.a[0] = {jac, jac_s_nz, jac_s_inst};
+    A.n = n;
+    A.lds = round_up(n, 64);
+    if (parts_map_jac(j, n, A, s)) return 0;
+  }
+  JitJac& J = jac_plan(j, n);
+  jac_build(j, J);
   const int64_t lds = round_up(n, 64);  // instances, padded to whole tiles of 64
   const int64_t homes = static_cast<int64_t>(J.n_group) * J.home_rows * lds;
   if (homes > 0) J.st.reserve(static_cast<size_t>(homes) * sizeof(double));
@@ -2446,6 +2451,7 @@ struct LinsolJit {
   cxh_tape_s tape;
   cxh_jac_s jac;
   int nrhs = 0;
+  int builds = -1;  // jit_linsol_builds, once known
   DeviceBuffer cnt;
 };
 
@@ -2687,6 +2693,19 @@ int jit_linsol_solve(LinsolJit& L, int64_t n_inst, const double* const* fac, int
   arg.a[n_fac] = {x, x_s, x_t};
   res.a[0] = {x, x_s, x_t};
   return jit_map_jac(&L.jac, n_inst, arg, res, nullptr, 0, 0, s);
+}
+
+bool jit_linsol_builds(LinsolJit& L) {
+  if (L.builds < 0 && no_alloc_active()) return true;  // nothing compiles now: the launch says so
+  if (L.builds < 0) {
+    try {
+      jac_build(&L.jac, jac_plan(&L.jac, 1));
+      L.builds = 1;
+    } catch (const std::runtime_error&) {
+      L.builds = 0;
+    }
+  }
+  return L.builds == 1;
 }
 
 std::string jit_linsol_source(LinsolJit& L, int segment) {

@@ -433,16 +433,38 @@ struct cxh_qr_s {
   DeviceBuffer cmp_flag;
 };
 
-// Largest batch of the sixteen-lane programs (CXH_LINSOL_ROWS_MAX overrides).
-// They spend about four times the instructions of the one-lane programs per
-// instance on four times the wavefronts: ahead while the one-lane programs
-// leave SIMDs idle, behind once those fill the chip.  Horizon-30 KKT, us per
-// call, sixteen-lane / one-lane: LDL 141 / 333 at 8192 instances, 285 / 434 at
-// 16384, 573 / 585 at 32768, 877 / 772 at 49152; QR 271 / 805, 602 / 927,
-// 1132 / 1251, 1613 / 1558.
-static int64_t rows_max() {
-  if (const char* e = std::getenv("CXH_LINSOL_ROWS_MAX")) return std::atoll(e);
-  return 32768;
+// The one-lane programs: of LDL part `part` (nrhs: fused), of the fused QR, of
+// the QR's factor.
+static sxh::LinsolJit& ldl_program(cxh_ldl_s* l, int part, int nrhs) {
+  auto& J = part == LS_FUSED ? l->jit[nrhs] : part == LS_FACTOR ? l->jit_fact : l->jit_solve;
+  if (!J)
+    J = sxh::jit_ldl_create(l->lt.ncol, l->a.colind, l->a.row, l->lt.colind, l->lt.row, l->p,
+                            part == LS_FUSED ? nrhs : part == LS_FACTOR ? 0 : 1, part);
+  return *J;
+}
+
+static sxh::LinsolJit& qr_program(cxh_qr_s* q, int nrhs, bool tr) {
+  auto& J = q->jit[2 * nrhs + (tr ? 1 : 0)];
+  if (!J)
+    J = sxh::jit_qr_create(q->a.ncol, q->v.nrow, q->a.colind, q->a.row, q->v.colind, q->v.row, q->r.colind,
+                           q->r.row, q->prinv, q->pc, q->eps, nrhs, tr);
+  return *J;
+}
+
+static sxh::LinsolJit& qr_factor_program(cxh_qr_s* q) {
+  if (!q->jit_fact)
+    q->jit_fact = sxh::jit_qr_create(q->a.ncol, q->v.nrow, q->a.colind, q->a.row, q->v.colind, q->v.row, q->r.colind,
+                                     q->r.row, q->prinv, q->pc, q->eps, 0, false, LS_FACTOR);
+  return *q->jit_fact;
+}
+
+// Whether a sixteen-lane program serves a batch: up to its own limit
+// (RowsProgram::limit; CXH_LINSOL_ROWS_MAX in its place), and up to kRowsMost
+// where the one-lane program cannot be built without scratch.
+template <class F>
+static bool rows_serve(const sxh::RowsProgram& P, int64_t n_inst, F&& one_lane) {
+  if (const char* e = std::getenv("CXH_LINSOL_ROWS_MAX")) return n_inst <= std::atoll(e);
+  return n_inst <= P.limit || (n_inst <= sxh::kRowsMost && !sxh::jit_linsol_builds(one_lane()));
 }
 
 // 32-bit byte strides and offsets: a row of n_inst doubles, the kept blocks.
@@ -464,10 +486,11 @@ static sxh::RowsProgram* ldl_rows_program(cxh_ldl_s* l, int part) {
 // The sixteen-lane program that serves a call, compiled; null: the one-lane
 // programs serve it.
 static sxh::RowsProgram* ldl_rows(cxh_ldl_s* l, int part, int64_t n_inst) {
-  if (n_inst > rows_max()) return nullptr;
   sxh::RowsProgram* P = ldl_rows_program(l, part);
-  if (P && !rows_fit(*P, n_inst)) return nullptr;
-  if (P && !sxh::rows_ready(*P)) {
+  if (!P || !rows_fit(*P, n_inst) ||
+      !rows_serve(*P, n_inst, [&]() -> sxh::LinsolJit& { return ldl_program(l, part, 1); }))
+    return nullptr;
+  if (!sxh::rows_ready(*P)) {
     l->rows[part].reset();
     P = nullptr;
   }
@@ -486,10 +509,11 @@ static sxh::RowsProgram* qr_rows_program(cxh_qr_s* q, int part) {
 }
 
 static sxh::RowsProgram* qr_rows(cxh_qr_s* q, int part, int64_t n_inst) {
-  if (n_inst > rows_max()) return nullptr;
   sxh::RowsProgram* P = qr_rows_program(q, part);
-  if (P && !rows_fit(*P, n_inst)) return nullptr;
-  if (P && !sxh::rows_ready(*P)) {
+  if (!P || !rows_fit(*P, n_inst) ||
+      !rows_serve(*P, n_inst, [&]() -> sxh::LinsolJit& { return part == LS_FUSED ? qr_program(q, 1, false) : qr_factor_program(q); }))
+    return nullptr;
+  if (!sxh::rows_ready(*P)) {
     q->rows[part].reset();
     P = nullptr;
   }
@@ -509,14 +533,6 @@ static int rows_text(const sxh::RowsProgram* P, char* buf, int64_t cap, int64_t*
   }
   if (tab && m) std::memcpy(tab, P->tab.data(), static_cast<size_t>(std::min(m, tab_cap)) * sizeof(int32_t));
   return 0;
-}
-
-static sxh::LinsolJit& qr_program(cxh_qr_s* q, int nrhs, bool tr) {
-  auto& J = q->jit[2 * nrhs + (tr ? 1 : 0)];
-  if (!J)
-    J = sxh::jit_qr_create(q->a.ncol, q->v.nrow, q->a.colind, q->a.row, q->v.colind, q->v.row, q->r.colind,
-                           q->r.row, q->prinv, q->pc, q->eps, nrhs, tr);
-  return *J;
 }
 
 static void upload_ints(DeviceBuffer& b, const std::vector<int>& v) {
@@ -642,9 +658,7 @@ int cxh_ldl_factor_solve(cxh_ldl l, int64_t n_inst, const double* a, double* x, 
       sxh::rows_launch(*R, n_inst, io, static_cast<hipStream_t>(stream));
       return 0;
     }
-    auto& J = l->jit[nrhs];
-    if (!J) J = jit_ldl_create(n, l->a.colind, l->a.row, l->lt.colind, l->lt.row, l->p, nrhs);
-    return jit_linsol_run(*J, n_inst, a, soa ? n_inst : 1, soa ? 1 : nnz_a, x, soa ? n_inst : 1,
+    return jit_linsol_run(ldl_program(l, LS_FUSED, nrhs), n_inst, a, soa ? n_inst : 1, soa ? 1 : nnz_a, x, soa ? n_inst : 1,
                        soa ? 1 : static_cast<int64_t>(n) * nrhs, status, static_cast<hipStream_t>(stream));
   }
   ldl_generic(l, LS_FUSED, n_inst, a, x, nrhs, status, layout, static_cast<hipStream_t>(stream));
@@ -683,9 +697,8 @@ int cxh_ldl_nfact(cxh_ldl l, int64_t n_inst, const double* a, int32_t* status, i
       l->fact_n = n_inst;
       return 0;
     }
-    if (!l->jit_fact) l->jit_fact = jit_ldl_create(n, l->a.colind, l->a.row, l->lt.colind, l->lt.row, l->p, 0,
-                                                   LS_FACTOR);
-    if (int rc = jit_linsol_factor(*l->jit_fact, n_inst, a, soa ? n_inst : 1, soa ? 1 : nnz_a, fac, 2, ld, status, s))
+    if (int rc = jit_linsol_factor(ldl_program(l, LS_FACTOR, 0), n_inst, a, soa ? n_inst : 1, soa ? 1 : nnz_a, fac, 2, ld,
+                                   status, s))
       return rc;
   } else {
     ldl_generic(l, LS_FACTOR, n_inst, a, nullptr, 0, status, layout, s);
@@ -726,12 +739,11 @@ int cxh_ldl_solve(cxh_ldl l, int64_t n_inst, double* x, int32_t nrhs, int32_t tr
       }
       return 0;
     }
-    auto& J = l->jit_solve;
-    if (!J) J = jit_ldl_create(n, l->a.colind, l->a.row, l->lt.colind, l->lt.row, l->p, 1, LS_SOLVE);
+    sxh::LinsolJit& J = ldl_program(l, LS_SOLVE, 1);
     // the right-hand sides one after another: each is solved on its own, in
     // the order the fused program solves it, so the bits are the same
     for (int q = 0; q < nrhs; ++q)
-      if (int rc = jit_linsol_solve(*J, n_inst, fac, 2, ld, x + static_cast<int64_t>(q) * n * (soa ? n_inst : 1),
+      if (int rc = jit_linsol_solve(J, n_inst, fac, 2, ld, x + static_cast<int64_t>(q) * n * (soa ? n_inst : 1),
                                     soa ? n_inst : 1, soa ? 1 : static_cast<int64_t>(n) * nrhs, s))
         return rc;
     return 0;
@@ -771,9 +783,7 @@ int cxh_ldl_jit_source(cxh_ldl l, int32_t nrhs, char* buf, int64_t cap, int64_t*
   CXH_TRY
   if (!l) return cxh_fail("null ldl handle");
   if (nrhs < 0) return cxh_fail("negative nrhs");
-  auto& J = l->jit[nrhs];
-  if (!J) J = jit_ldl_create(l->lt.ncol, l->a.colind, l->a.row, l->lt.colind, l->lt.row, l->p, nrhs);
-  const std::string src = jit_linsol_source(*J, 0);
+  const std::string src = jit_linsol_source(ldl_program(l, LS_FUSED, nrhs), 0);
   if (len) *len = static_cast<int64_t>(src.size());
   if (buf && cap > 0) {
     const size_t m = std::min<size_t>(src.size(), static_cast<size_t>(cap - 1));
@@ -1073,11 +1083,8 @@ int cxh_qr_nfact(cxh_qr q, int64_t n_inst, const double* a, int32_t* status, int
       io.status = st;
       io.eps = q->eps;
       sxh::rows_launch(*R, n_inst, io, s);
-    } else {
-    if (!q->jit_fact)
-      q->jit_fact = jit_qr_create(q->a.ncol, q->v.nrow, q->a.colind, q->a.row, q->v.colind, q->v.row, q->r.colind,
-                                  q->r.row, q->prinv, q->pc, q->eps, 0, false, LS_FACTOR);
-    if (int rc = jit_linsol_factor(*q->jit_fact, n_inst, a, soa ? n_inst : 1, soa ? 1 : nnz_a, fac, 3, ld, st, s))
+    } else if (int rc = jit_linsol_factor(qr_factor_program(q), n_inst, a, soa ? n_inst : 1, soa ? 1 : nnz_a, fac, 3, ld, st,
+                                          s)) {
       return rc;
     }
   } else {

@@ -319,7 +319,7 @@ void finish(RowsEmit& E, const std::string& decl, const std::string& tail, RowsP
   }
   unsigned staged = 0;
   for (int w : E.entry) staged |= 1u << (static_cast<unsigned>(w) >> 29);
-  std::string o = "#define CXR_STAGED " + S(staged) + "\n";
+  std::string o = "// batches up to " + S(P.limit) + "\n#define CXR_STAGED " + S(staged) + "\n";
   o += kRowsPrologue;
   o += "CXR_BODY(cxr_body) {\n  CXR_SETUP();\n" + decl;
   for (int j = 0; j < kFlight; ++j) o += "  vd s" + S(j) + " = 0.0;\n";
@@ -334,6 +334,28 @@ void finish(RowsEmit& E, const std::string& decl, const std::string& tail, RowsP
   P.source = std::move(o);
   P.tab = std::move(E.entry);
   P.tab.insert(P.tab.end(), E.rows.begin(), E.rows.end());
+}
+
+// Largest batch of a program whose pivots hold `values` values in all, `wide`
+// a pivot or more being worth kRowsMost.  The sixteen-lane programs spend the
+// same instructions on a pivot however many of the lanes hold something, on four
+// times the wavefronts: ahead while the one-lane programs leave SIMDs idle,
+// behind once those fill the chip, and the sooner the fewer values there are.
+// 274 rows, us per call, sixteen-lane / one-lane:
+//   LDL factor + solve, 2.0 values a pivot (tridiagonal): 103 / 124 at 8192
+//   instances, 133 / 126 at 12288, 319 / 237 at 32768; 3.0: 157 / 164 at 12288,
+//   186 / 175 at 14336; 5.0: 262 / 304 at 16384, 479 / 421 at 32768; 6.7 (control
+//   KKT): 155 / 336 at 8192, 537 / 576 at 32768; 8.9: 696 / 810 at 32768
+//   LDL factor alone: 2.0: 96 / 96 at 12288; 5.0: 205 / 280 at 16384, 375 / 336
+//   at 32768; 6.7: 439 / 489 at 32768
+//   LDL solve alone (little to do per pivot): 2.0: 82 / 98 at 8192, 102 / 98 at
+//   10240; 5.0: 167 / 167 at 12288, 235 / 195 at 16384; 6.7: 197 / 242 at 12288,
+//   566 / 393 at 32768
+//   QR factor + solve, 6.0: 372 / 434 at 16384, 677 / 606 at 32768 (factor alone
+//   355 / 506, 643 / 620); 9.9: 876 / 989 at 32768; 12.0 (control KKT): 1132 / 1251 at 32768, 1613 / 1558 at 49152
+int64_t batch_limit(int64_t values, int pivots, double wide, int64_t most) {
+  const double per_pivot = static_cast<double>(values) / pivots;
+  return std::min(most, per_pivot >= wide ? kRowsMost : static_cast<int64_t>(4096 * per_pivot));
 }
 
 using Idx = std::vector<int>;
@@ -532,6 +554,7 @@ bool rows_ldl_source(int n, const std::vector<int>& a_colind, const std::vector<
   }
   P.kernel = part == LS_FUSED ? "cxj_ldl_rows" : part == LS_FACTOR ? "cxj_ldl_rows_fact" : "cxj_ldl_rows_solve";
   P.kept = solve ? block[n] : 0;
+  P.limit = batch_limit(block[n], n, 6.0, part == LS_SOLVE ? 12288 : kRowsMost);
   finish(E, decl, factor ? "  CXR_COUNT(cnt);\n" : "", P);
   return true;
 }
@@ -746,6 +769,7 @@ bool rows_qr_source(int ncol, int nrow, const std::vector<int>& a_colind, const 
   for (int s = 0; s < n_slot; ++s) decl += "  vd x_" + S(s) + " = 0.0;\n";
   P.kernel = solve ? "cxj_qr_rows" : "cxj_qr_rows_fact";
   P.kept = solve ? block[ncol] : 0;
+  P.limit = batch_limit(block[ncol] + (solve ? 0 : ncol), ncol, 8.0, kRowsMost);  // the right-hand side's lane in both
   finish(E, decl, "  CXR_COUNT(cnt);\n", P);
   return true;
 }

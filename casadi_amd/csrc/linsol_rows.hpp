@@ -10,12 +10,15 @@
 
 namespace sxh {
 
+constexpr int64_t kRowsMost = 32768;  // no sixteen-lane program serves a larger batch
+
 // A generated program, its index table and, once compiled, its kernel.
 struct RowsProgram {
   const char* kernel = "";
   std::string source;
   std::vector<int> tab;
   int64_t kept = 0;  // doubles per instance kept between the sweeps (RowsIO::w)
+  int64_t limit = 0;  // largest batch it serves by choice (batch_limit)
   DeviceBuffer d_tab;
   hipFunction_t fn = nullptr;
 };

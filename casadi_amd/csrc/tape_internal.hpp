@@ -212,6 +212,8 @@ int jit_linsol_factor(LinsolJit& L, int64_t n_inst, const double* a, int64_t a_s
 // The solve program: factor blocks fac[b] ([rows][ld]), x overwritten in place.
 int jit_linsol_solve(LinsolJit& L, int64_t n_inst, const double* const* fac, int n_fac, int64_t ld, double* x,
                      int64_t x_s, int64_t x_t, hipStream_t s);
+// Compiles the program; false when no register budget keeps it off scratch.
+bool jit_linsol_builds(LinsolJit& L);
 std::string jit_linsol_source(LinsolJit& L, int segment);
 int jit_linsol_segments(LinsolJit& L);
 }

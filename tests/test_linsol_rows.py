@@ -183,6 +183,24 @@ def test_wide_patterns_keep_the_one_lane_program():
     assert Linsol("q", "qr", W.ocp_kkt_sparsity(3, 6, 3)[0]).rows_source(0) is None
 
 
+def test_batch_limit_follows_the_width():
+    """A pattern whose pivots hold few values leaves the sixteen lanes at a
+    smaller batch: 4096 instances per value, all 32768 from 6 (LDL) or 8 (QR)
+    values, the LDL's solve alone at most 12288."""
+    from casadi_amd import workloads as W
+    from casadi_amd.linsol import Linsol
+    from casadi_amd.sx import Sparsity
+    i = np.arange(39)
+    d = np.arange(40)
+    tri = Sparsity.triplet(40, 40, np.concatenate([d, i, i + 1]), np.concatenate([d, i + 1, i]))
+    kkt = W.ocp_kkt_sparsity(30)[0]
+    limit = lambda solver, sp, part: int(Linsol("l", solver, sp, {"amd": sp is kkt}).rows_source(part)[0].split("\n")[0].split()[-1])
+    assert [limit("ldl", tri, p) for p in (0, 1, 2)] == [4096 * 79 // 40] * 3
+    assert [limit("qr", tri, p) for p in (0, 1)] == [4096 * (3 * 40 - 3 + 40) // 40] * 2
+    assert [limit("ldl", kkt, p) for p in (0, 1, 2)] == [32768, 32768, 12288]
+    assert [limit("qr", kkt, p) for p in (0, 1)] == [32768, 32768]
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("solver", ["ldl", "qr"])
 @pytest.mark.parametrize("n_inst", [1, 15, 16, 17, 63, 65, 1000])
@@ -209,3 +227,28 @@ def test_rows_programs_match_the_generic_kernel(cuda, monkeypatch, solver, n_ins
     monkeypatch.setenv("CXH_LINSOL_ROWS_MAX", "0")
     xo, so = Linsol("o", solver, sp).solve_batch(A, B)
     assert torch.equal(so, sr) and np.array_equal(xo.cpu().numpy(), xr.cpu().numpy(), equal_nan=True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("solver", ["ldl", "qr"])
+def test_one_lane_programs_match_the_generic_kernel(cuda, monkeypatch, solver):
+    """The horizon-30 system through the programs that batches above the
+    sixteen-lane limit run (several segments for the QR): fused, factor alone
+    and solve alone."""
+    import torch
+    from casadi_amd import workloads as W
+    from casadi_amd.linsol import Linsol
+    monkeypatch.setenv("CXH_LINSOL_ROWS_MAX", "0")
+    n_inst = 193
+    sp, a = W.ocp_kkt_batch(np.random.default_rng(30), n_inst, 30)
+    A = torch.tensor(a, device="cuda")
+    B = torch.tensor(np.random.default_rng(31).standard_normal((sp.size1(), n_inst)), device="cuda")
+    one, gen = Linsol("o", solver, sp), Linsol("i", solver, sp, {"engine": "interp"})
+    for s in (one, gen):
+        s.nfact(A)
+    print(f"[case] one-lane {solver} factor", flush=True)
+    assert torch.equal(one.solve(B), gen.solve(B))
+    print(f"[case] one-lane {solver} solve", flush=True)
+    for name in ("l", "again"):
+        (x, st), (xg, sg) = one.solve_batch(A, B), gen.solve_batch(A, B)
+        assert torch.equal(x, xg) and torch.equal(st, sg), name
