@@ -2208,6 +2208,12 @@ struct JitParts {
 // (one wavefront per SIMD) share a CU's 160 KB.
 constexpr int kPartLdsRows = 80;
 
+// Device memory for spill rows past those (bytes): a unit needs its rows for
+// every instance of a launch, so larger batches go in several.  The quadrotor
+// Hessian with five directions per group (136 rows, 98 units) still runs 78
+// tiles at once, 7600 wavefronts.
+constexpr int64_t kPartSpill = int64_t(512) << 20;
+
 // outs: whether the outputs are stored (all of them or none).
 static std::string gen_parts_kernel(JitParts& P, int R, int group, bool soa32, bool outs, int* n_units, int* spill_rows) {
   std::string bodies, dispatch;
@@ -2325,8 +2331,12 @@ static bool parts_map_jac(cxh_jac_s* j, int64_t n, CxjArgs A, hipStream_t s) {
     K.spill_rows = ns;
   }
   if (K.units > 65535) return false;
+  // spill rows in device memory: as many tiles of 64 instances in one launch as kPartSpill holds
+  const int64_t tile = 64 * K.spill_rows * K.units * static_cast<int64_t>(sizeof(double));
+  if (tile > kPartSpill) return false;
+  const int64_t step = tile > 0 ? std::min<int64_t>(kPartSpill / tile * 64, A.lds) : A.lds;
   if (!P.d_rows.ptr) P.d_rows.upload(P.rows.data(), P.rows.size() * sizeof(int));
-  if (K.spill_rows > 0) P.spill.reserve(static_cast<size_t>(K.spill_rows * K.units * A.lds) * sizeof(double));
+  if (tile > 0) P.spill.reserve(static_cast<size_t>(tile * (step / 64)));
   for (auto& a : A.arg.a)  // an absent input reads zeros: one device zero, strides 0
     if (!a.p) {
       if (!P.zero.ptr) {
@@ -2336,11 +2346,19 @@ static bool parts_map_jac(cxh_jac_s* j, int64_t n, CxjArgs A, hipStream_t s) {
       a = {P.zero.as<double>(), 0, 0};
     }
   A.adj_in = P.d_rows.as<double>();  // the row table
-  A.spill = K.spill_rows > 0 ? P.spill.as<double>() : nullptr;
-  void* params[] = {&A};
-  hip_check(hipModuleLaunchKernel(K.fn, static_cast<unsigned>((n + 63) / 64), static_cast<unsigned>(K.units), 1, 64, 1, 1, 0,
-                                  s, params, nullptr),
-            "jit parts kernel launch");
+  A.spill = tile > 0 ? P.spill.as<double>() : nullptr;
+  A.lds = step;
+  for (int64_t k0 = 0; k0 < n; k0 += step) {
+    CxjArgs B = A;
+    B.n = std::min<int64_t>(step, n - k0);
+    for (IOTable* t : {&B.arg, &B.res, &B.asens})
+      for (auto& a : t->a)
+        if (a.p) a.p += k0 * a.s_inst;
+    void* params[] = {&B};
+    hip_check(hipModuleLaunchKernel(K.fn, static_cast<unsigned>((B.n + 63) / 64), static_cast<unsigned>(K.units), 1, 64, 1, 1,
+                                    0, s, params, nullptr),
+              "jit parts kernel launch");
+  }
   return true;
 }
 

@@ -194,3 +194,27 @@ def test_parts_keep_the_bits(cuda, monkeypatch, kind, n):
     assert none == [None] and torch.equal(jo, j)
     zeros = [args[0], torch.zeros_like(args[1])]
     assert torch.equal(h([args[0], None])[1], h(zeros)[1])
+
+
+@pytest.mark.gpu
+def test_parts_spill_memory_is_bounded(cuda, monkeypatch):
+    """Spill rows of a batch that would need more than half a GiB: several
+    launches over slices of the batch, the same bits."""
+    import torch
+    f, make = _plan("ocp4")
+    n = 40001
+    args = [torch.tensor(np.random.default_rng(n).uniform(-1, 1, (f.nnz_in(i), n)), device="cuda") for i in range(2)]
+    print(f"[case] parts spill n={n}", flush=True)
+    (y,), j = make(engine="jit")(args)
+    monkeypatch.setenv("CXH_JIT_TANREGS", "24")
+    h = make(engine="jit")
+    _, _, units, spill = h.parts_source()
+    assert units * spill * n * 8 > 2 << 29
+    y2, j2 = torch.empty_like(y), torch.empty_like(j)   # leaves torch two blocks of the results' sizes
+    del y2, j2
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    (ys,), js = h(args)
+    torch.cuda.synchronize()
+    assert before - torch.cuda.mem_get_info()[0] < 600 << 20
+    assert torch.equal(ys, y) and torch.equal(js, j)
