@@ -1532,6 +1532,13 @@ struct JitJac {
 // within the group (0: the primal).
 static int64_t home_key(int def, int dir_in_group) { return static_cast<int64_t>(def) * 128 + dir_in_group; }
 
+static int64_t device_simds() {
+  int dev = 0, cus = 0;
+  hip_check(hipGetDevice(&dev), "hipGetDevice");
+  hip_check(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev), "device CU count");
+  return 4 * static_cast<int64_t>(std::max(cus, 1));
+}
+
 // Directions per group.  Each group is a body of its own over all instances
 // (n/64 waves) and the kernels hold about one wave per SIMD (register-bound),
 // so by default the directions are split into as many groups as fill the
@@ -1540,12 +1547,8 @@ static int64_t home_key(int def, int dir_in_group) { return static_cast<int64_t>
 static int jac_dir_group(int ndir, int64_t n) {
   if (const char* e = std::getenv("CXH_JIT_DIRGROUP")) return std::max(1, std::atoi(e));
   if (n <= 0) return 8;
-  int dev = 0, cus = 0;
-  hip_check(hipGetDevice(&dev), "hipGetDevice");
-  hip_check(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev), "device CU count");
-  const int64_t simds = 4 * static_cast<int64_t>(std::max(cus, 1));
   const int64_t waves = std::max<int64_t>(1, (n + 63) / 64);
-  const int64_t groups = std::min<int64_t>(std::max<int64_t>(1, (simds + waves / 2) / waves), std::max(ndir, 1));
+  const int64_t groups = std::min<int64_t>(std::max<int64_t>(1, (device_simds() + waves / 2) / waves), std::max(ndir, 1));
   return static_cast<int>((ndir + groups - 1) / groups);
 }
 
@@ -1702,8 +1705,8 @@ static int jac_prefetch(const cxh_jac_s* j) {
 // part: the plan is a class of independent parts (PartClass), number `cls` of
 // its kernel.  A row that advances by a fixed step from part to part (stages
 // of a horizon) is computed from the part's number, any other comes from the
-// row table: a scalar load waited for at every use (245 of them
-// in the quadrotor stage's program).
+// row table, a scalar load waited for at every use: 6 rows of the quadrotor
+// Hessian's program, 245 with every row in the table.
 static std::string gen_tangent(const cxh_jac_s* j, const JitJac& J, int g, int s, int R, int* spill_rows,
                                const PartClass* part = nullptr, int cls = 0) {
   auto row = [&](int k) {
@@ -2201,7 +2204,7 @@ struct JitParts {
     hipFunction_t fn = nullptr;
     int64_t units = 0, spill_rows = 0;  // spill rows in device memory (0: in LDS, or none)
   };
-  std::map<std::array<int, 3>, Kernel> fn;  // by (directions per group, 32-bit offsets, outputs stored)
+  std::map<std::array<int, 3>, Kernel> fn;  // by (parts_build's `asked`, 32-bit offsets, outputs stored)
 };
 
 // Spill rows a block of 64 lanes keeps in LDS: 40 KB, so that four blocks
@@ -2269,16 +2272,41 @@ static bool parts_enabled() {
   return !(e && e[0] == '0') && !std::getenv("CXH_JIT_TANSEG");
 }
 
-// Directions per group of the parts' programs: each group computes the primal
-// again, and each direction more needs more values resident.  Quadrotor
-// Hessian (10 directions, horizon 20), us at 16384 / 1001 / 64 instances:
-// 3 directions 275 / 29 / 14 (49 spill rows, in LDS), 2: 294 / 26 / 14, 1: 465 /
-// 45 / 21, 5: 345 / 43 / 30 (135 spill rows, in device memory).  Register
-// budgets of 100-120 values (two wavefronts per SIMD) spill to device memory
-// as well: 470-530 us.
+// Directions per group of the parts' programs.  Each group computes the primal
+// again, and each direction more needs more values resident: few wavefronts want
+// small groups, many want large ones, unless the values no longer fit and spill to
+// device memory.  So there are as many groups as fill the SIMDs once (tiles of 64
+// instances x parts x groups), of at least three directions, and more where their
+// spill rows don't fit LDS.  us per call, by directions per group (d: spill rows
+// in device memory):
+//   quadrotor Hessian, 10 directions, 20 stages: 3: 15 / 27 / 256 / 1015 at 64 /
+//   1024 / 16384 / 65536 instances, 5d: 20 / 27 / 314 / 1217, 10d: 32 / 46 / 647 /
+//   2500, 1: 21 / 45 / 465 at the first three; whole tape 227 / 280 / 631 / 3230
+//   8 parts, dense in 24 directions: 3: 17 / 22 / 174 / 627, 12: 24 / 26 / 130 /
+//   505, 24: 504 at 65536; whole tape 253 at 16384, 553 at 65536
+//   4 parts, dense in 40 directions, at 4096 / 16384 / 60001 / 65536: 3: 79 / 259 /
+//   1222 / 1016, 10: 46 / 188 / 1098 / 978, 40: 78 / 202 / 1125 / 795; whole tape
+//   121 / 255 / 1234 / 738 (3.4 GB of stores: 650 us)
+// Register budgets of 100-120 values (two wavefronts per SIMD) spill to device
+// memory as well: 470-530 us for the Hessian at 16384.
+constexpr int kPartGroup = 3;
+
 static int parts_dir_group() {
   if (const char* e = std::getenv("CXH_JIT_DIRGROUP")) return std::max(1, std::atoi(e));
-  return 3;
+  return kPartGroup;
+}
+
+// Number of direction groups that n instances ask for.
+static int parts_groups(const JitParts& P, int64_t n) {
+  int nd = 1;
+  int64_t parts = 0;
+  for (const auto& c : P.cls) {
+    nd = std::max(nd, c->jac.ndir);
+    parts += c->count;
+  }
+  const int64_t most = (nd + kPartGroup - 1) / kPartGroup;
+  const int64_t waves = std::max<int64_t>(1, (n + 63) / 64) * std::max<int64_t>(1, parts);
+  return static_cast<int>(std::min(std::max<int64_t>(1, (device_simds() + waves / 2) / waves), most));
 }
 
 static int parts_reg_budget() {
@@ -2301,6 +2329,29 @@ static bool all_soa(const IOTable& t, size_t n) {
   return true;
 }
 
+// The kernel of the fewest groups, from `asked` on, whose spill rows fit LDS; of
+// groups of kPartGroup directions (asked < 0: of -asked) whatever they spill.  K.fn stays null where no register budget avoids scratch.
+static void parts_build(JitParts& P, int asked, bool soa, bool outs, JitParts::Kernel& K) {
+  int nd = 1;
+  for (const auto& c : P.cls) nd = std::max(nd, c->jac.ndir);
+  for (int g = asked;; ++g) {
+    const int group = asked < 0 ? -asked : std::max((nd + g - 1) / g, kPartGroup);
+    const bool last = asked < 0 || group == kPartGroup;
+    for (int R = parts_reg_budget(); R >= 24; R -= 24) {
+      int units = 0, ns = 0;
+      const std::string src = gen_parts_kernel(P, R, group, soa, outs, &units, &ns);
+      if (ns > 0 && !last) break;
+      hipFunction_t f = jit_function(src, "cxj_parts");
+      if (scratch_bytes(f) > 0) continue;
+      K.fn = f;
+      K.units = units;
+      K.spill_rows = ns;
+      return;
+    }
+    if (last) return;
+  }
+}
+
 // The sweep over the parts of the tape; false when it does not split (or the
 // kernel would need scratch) and the whole tape's kernels serve the call.
 static bool parts_map_jac(cxh_jac_s* j, int64_t n, CxjArgs A, hipStream_t s) {
@@ -2314,21 +2365,14 @@ static bool parts_map_jac(cxh_jac_s* j, int64_t n, CxjArgs A, hipStream_t s) {
   if (!A.asens.a[0].p || (have != 0 && have != blocks)) return false;
   JitParts& P = parts_of(j);
   if (P.cls.empty()) return false;
-  const int group = parts_dir_group();
+  const int asked = std::getenv("CXH_JIT_DIRGROUP") ? -parts_dir_group() : parts_groups(P, n);
   const bool soa = static_cast<uint64_t>(n) * 8u < (uint64_t(1) << 32) && A.asens.a[0].s_inst == 1 &&
                    all_soa(A.arg, j->tape->nnz_in.size()) && all_soa(A.res, j->tape->nnz_out.size());
-  JitParts::Kernel& K = P.fn[{group, soa ? 1 : 0, have ? 1 : 0}];
-  for (int R = parts_reg_budget(); !K.fn; R -= 24) {
-    if (R < 24) {
-      P.cls.clear();
-      return false;
-    }
-    int units = 0, ns = 0;
-    hipFunction_t f = jit_function(gen_parts_kernel(P, R, group, soa, have != 0, &units, &ns), "cxj_parts");
-    if (scratch_bytes(f) > 0) continue;
-    K.fn = f;
-    K.units = units;
-    K.spill_rows = ns;
+  JitParts::Kernel& K = P.fn[{asked, soa ? 1 : 0, have ? 1 : 0}];
+  if (!K.fn) parts_build(P, asked, soa, have != 0, K);
+  if (!K.fn) {
+    P.cls.clear();
+    return false;
   }
   if (K.units > 65535) return false;
   // spill rows in device memory: as many tiles of 64 instances in one launch as kPartSpill holds

@@ -11,9 +11,9 @@
 //
 // Here the tape is taken apart into those sets.  Parts whose instructions,
 // constants, seeds and scatter agree up to the rows they touch are one class:
-// one program, run side by side over instances and parts, reading the rows of
-// its inputs, outputs and nonzeros from a table indexed by the part
-// (wave-uniform scalar loads).  Every value is computed by the same operations
+// one program, run side by side over instances and parts.  The rows of its
+// inputs, outputs and nonzeros are computed from the part's number where they
+// advance by a fixed step from part to part, and read from a table where not.  Every value is computed by the same operations
 // on the same operands as before, so the bits do not change.
 //
 // Measured, quadrotor Lagrangian Hessian, whole-tape kernels / parts: horizon
@@ -239,8 +239,8 @@ std::vector<std::unique_ptr<PartClass>> find_parts(const cxh_jac_s* j, std::vect
     return work(x) != work(y) ? work(x) > work(y) : x[0] < y[0];
   });
   // Worth it when the longest part is at most half of the tape: the parts run
-  // side by side, so that is what the chain of one instance shrinks to (and
-  // the code never grows).  Many classes are many programs in one kernel.
+  // side by side, so that is what the chain of one instance shrinks to.  Many
+  // classes are many programs in one kernel.
   int64_t longest = 0, ops = 0;
   for (const auto& g : groups) {
     longest = std::max(longest, static_cast<int64_t>(parts[g[0]].instr.size()));

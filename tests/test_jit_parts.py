@@ -36,6 +36,19 @@ def _stages(n_stage, irregular=False, aux=False):
     return ca.Function("stages", [x, p], [ca.vertcat(*out)])
 
 
+def _dense(n_part, width):
+    """f: per part a map of `width` inputs to as many outputs, each depending on all of them."""
+    import casadi_amd as ca
+    x = ca.SX.sym("x", n_part * width)
+    out = []
+    for p in range(n_part):
+        v = [x[width * p + i] for i in range(width)]
+        h = [ca.sin(v[i]) * v[(i + 1) % width] for i in range(width)]
+        s = sum(0.7 * e for e in h)
+        out += [ca.cos(s + v[i]) * h[i] + v[i] / 1.1 for i in range(width)]
+    return ca.Function("dense", [x], [ca.vertcat(*out)])
+
+
 def _plan(kind):
     import casadi_amd as ca
     from casadi_amd import workloads as W
@@ -44,6 +57,9 @@ def _plan(kind):
         w, lam, lag = W.quadrotor_ocp_lagrangian(N=int(kind[3:]))
         f = ca.Function("grad_lag", [w, lam], [ca.gradient(lag, w)])
         return f, lambda **k: HipJacobian(f, symmetric=True, first_block=True, **k)
+    if kind.startswith("dense"):
+        f = _dense(12, int(kind[5:]))
+        return f, lambda **k: HipJacobian(f, **k)
     f = _stages(40 if kind == "regular" else 41, kind == "irregular", kind != "regular")
     return f, lambda **k: HipJacobian(f, first_block=True, **k)
 
@@ -166,6 +182,29 @@ def test_an_output_written_twice_keeps_the_order():
     outs = np.flatnonzero(prog["op"] == OP.OUTPUT)
     prog["i2"][outs[-1]] = prog["i2"][outs[0]]
     assert HipJacobian(f, tape=tape(prog), first_block=True).parts_source() is None
+
+
+@pytest.mark.parametrize("size", ["5", "12"])
+def test_larger_direction_groups_on_host(monkeypatch, tmp_path, size):
+    """The group sizes that larger batches run, through the setting."""
+    monkeypatch.setenv("CXH_JIT_DIRGROUP", size)
+    test_parts_kernel_on_host(monkeypatch, tmp_path, "ocp4", "200", True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 2000, 5000, 20001])
+def test_group_sizes_keep_the_bits(cuda, monkeypatch, n):
+    """Batches of 12 parts dense in 14 directions that take groups of 3, of 5 and
+    (past the number of wavefronts that fills the device) of all 14."""
+    import torch
+    f, make = _plan("dense14")
+    x = torch.tensor(np.random.default_rng(n).uniform(-1, 1, (f.nnz_in(0), n)), device="cuda")
+    print(f"[case] parts groups n={n}", flush=True)
+    h = make(engine="jit")
+    assert h.parts_source() is not None
+    (y,), j = h([x])
+    (yi,), ji = make()([x])
+    assert torch.equal(y, yi) and torch.equal(j, ji)
 
 
 @pytest.mark.gpu
