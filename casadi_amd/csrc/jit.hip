@@ -482,7 +482,7 @@ static std::string adj_name(int64_t c, int64_t ws) {
 // sxh_div_c and take sin/cos without a branch, hold every output and
 // sensitivity back to the end (an output may be written over an input), and
 // evaluate again with `<name>_x`, which divides as IEEE 754 does and calls the
-// library's sincos past 2^20, when a lane of the wavefront reported an operand
+// library's sincos past 2^26, when a lane of the wavefront reported an operand
 // outside their ranges; *div counts the divisions and pairs.  cold: that exact
 // body, whose sin/cos sites do not count towards trig_call_sites().  The body is bound
 // by the instructions it issues (with few instances, by its chain), and an IEEE division is

@@ -652,7 +652,7 @@ std::string gen_functions(const cxh_tape_s* t, const RollPlan& L, bool rev, int6
     o += "}\n";
   }
   // The iteration functions: `_x` divides as IEEE 754 does and branches to
-  // the library's sin/cos past 2^20; when the body divides by constants or
+  // the library's sin/cos past 2^26; when the body divides by constants or
   // takes a sin or cos, `_f` divides through sxh_div_c, takes them without a
   // branch and reports in `wide` an operand outside their ranges (the loops
   // then run again with `_x`, see gen_roll).  One wave per SIMD waits for the

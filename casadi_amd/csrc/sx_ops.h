@@ -260,13 +260,13 @@ SXH_HD double sxh_div_c(double x, double c, double ci, W& wide) {
 }
 #endif
 
-// sin(x) and cos(x) for |x| <= 2^20 (either sign of zero kept).
+// sin(x) and cos(x) for |x| <= 2^26 (either sign of zero kept).
 //
 // Cody-Waite reduction with FMAs (W. J. Cody, W. Waite, "Software Manual for
 // the Elementary Functions", 1980): k = x * 2/pi rounded to an integer by the
 // addition of 1.5 * 2^52, whose low word then holds k; pi/2 = P1 + P2 + P3 with
-// 53, 33 and 53 bits.  x - k P1 is exact (a multiple of 2^-53 below 1), and so
-// is what its difference r to k P2 (a multiple of 2^-87, |k| < 2^20) rounds
+// 53, 27 and 53 bits.  x - k P1 is exact (a multiple of 2^-53 below 1), and so
+// is what its difference r to k P2 (a multiple of 2^-80, |k| < 2^26) rounds
 // off, so the reduced argument is r + rl with rl that remainder and the P3
 // term.  Then minimax polynomials on |r| <= pi/4 (Remez; with their rounded
 // coefficients within 2^-56.5 of sin and 2^-59.3 of cos, relatively), the leading
@@ -277,21 +277,25 @@ SXH_HD double sxh_div_c(double x, double c, double ci, W& wide) {
 // Error: the sine at |r| = pi/4 is the worst, 0.5 ulp for the last addition, 0.11
 // for r^2 and r^3 rounded in r^3 / 6, 0.07 for the roundings of what is
 // subtracted and 0.06 for the polynomial, 0.74 in all.  Over 100 million
-// arguments in each of +-0.8, +-1, +-10, +-1000 and +-2^20, against a 64-bit
-// significand: at most 0.726, mean 0.2509.  The device library's sincos, which
+// arguments in each of +-0.8, +-1, +-10, +-1000, +-2^20, +-2^24 and +-2^26, against
+// a 64-bit significand: at most 0.726, mean 0.2509; at the arguments nearest to
+// multiples of pi/2 (down to 2^-60) at most 0.5.  The device library's sincos, which
 // it replaces, over 800 000 arguments: at most 0.768, mean 0.2541.  About as many instructions as the
 // library's (45 against 48 per pair), but a shorter dependent chain, which is
 // what kernels with one wave per SIMD wait for: a 100-step cart-pole rollout's
 // gradient over 32768 instances 319 -> 295 us, the Hessian of 20 stages over
 // 16384 249 -> 238 us, the issue-bound map over 8388608 162 -> 156 us.
+// Past 2^26 a straight-line body runs twice (its flag, see gen_body in jit.hip),
+// twice the time of the library's two-step reduction alone: the range is the
+// largest that the three parts give.
 SXH_HD void sxh_sincos_reduced(double x, double* s, double* c) {
   const double m = 0x1.8p52;
   const double t = fma(x, 0x1.45f306dc9c883p-1, m);
   const unsigned k = static_cast<unsigned>(__builtin_bit_cast(unsigned long long, t));
   const double n = t - m;
   const double r0 = fma(n, -0x1.921fb54442d18p+0, x);
-  const double r = fma(n, -0x1.1a62633100000p-54, r0);
-  const double rl = fma(n, -0x1.1701b839a2520p-88, fma(n, -0x1.1a62633100000p-54, r0 - r));
+  const double r = fma(n, -0x1.1a62634p-54, r0);
+  const double rl = fma(n, 0x1.d747f23e32ed7p-83, fma(n, -0x1.1a62634p-54, r0 - r));
   const double z = r * r, v = z * r, zl = fma(r, r, -z);
   const double p = fma(fma(fma(fma(0x1.5d8ee78d06142p-33, z, -0x1.ae5e5780fa258p-26), z, 0x1.71de3564086f0p-19), z,
                            -0x1.a01a019bf9b5bp-13), z, 0x1.111111110f7b0p-7);
@@ -310,27 +314,27 @@ SXH_HD void sxh_sincos_reduced(double x, double* s, double* c) {
 
 // sin(x) and cos(x) from one argument reduction on the device, every engine
 // alike: the pair, and either of the two alone, have the same bits wherever
-// they are computed.  Arguments past 2^20, infinities and NaN take the
+// they are computed.  Arguments past 2^26, infinities and NaN take the
 // library's.  Two library calls on the host.
 SXH_HD void sxh_sincos(double x, double* s, double* c) {
 #if defined(__HIPCC_RTC__) || defined(__HIP_DEVICE_COMPILE__)
   sxh_sincos_reduced(x, s, c);
-  if (__builtin_expect(!(fabs(x) <= 0x1p20), 0)) sincos(x, s, c);
+  if (__builtin_expect(!(fabs(x) <= 0x1p26), 0)) sincos(x, s, c);
 #else
   *s = sin(x);
   *c = cos(x);
 #endif
 }
-// The pair without a branch: a finite |x| past 2^20 (and an infinity) sets
+// The pair without a branch: a finite |x| past 2^26 (and an infinity) sets
 // `wide`, and the caller then evaluates again with sxh_sincos.  NaN in, NaN out.
 template <class W>
 SXH_HD void sxh_sincos(double x, double* s, double* c, W& wide) {
 #if defined(__HIPCC_RTC__) || defined(__HIP_DEVICE_COMPILE__)
   sxh_sincos_reduced(x, s, c);
-  sxh_flag(fabs(x) > 0x1p20, wide);
+  sxh_flag(fabs(x) > 0x1p26, wide);
 #else
   sxh_sincos(x, s, c);
-  sxh_flag(fabs(x) > 0x1p20, wide);
+  sxh_flag(fabs(x) > 0x1p26, wide);
 #endif
 }
 SXH_HD double sxh_sin(double x) {

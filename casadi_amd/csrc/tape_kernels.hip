@@ -243,7 +243,7 @@ __device__ __forceinline__ int2 ximm(const int2& v, int j) {
 }
 __device__ __forceinline__ void xsincos(double x, double* s, double* c) {
   sxh_sincos_reduced(x, s, c);
-  if (__builtin_amdgcn_ballot_w64(!(fabs(x) <= 0x1p20))) {
+  if (__builtin_amdgcn_ballot_w64(!(fabs(x) <= 0x1p26))) {
     const SinCos r = sxh_sincos_call(x);
     *s = r.s;
     *c = r.c;

@@ -36,10 +36,10 @@ def _build(src, name, tmp):
 
 def _states(n, seed):
     """Cart-pole states and forces; of every ten instances one has angles past
-    2^20, one a speed whose tenth is below 2^-900 (and a zero angle)."""
+    2^26, one a speed whose tenth is below 2^-900 (and a zero angle)."""
     rng = np.random.default_rng(seed)
     x, u = rng.uniform(-1, 1, (4, n)), rng.uniform(-10, 10, (1, n))
-    x[:, 3::10] *= 4e6
+    x[:, 3::10] = np.copysign(2e8, x[:, 3::10])
     x[:, 7::10] *= 1e-300
     u[:, 7::10] *= 1e-300
     return x, u, np.isin(np.arange(n) % 10, (3, 7))

@@ -42,11 +42,18 @@ def reduced(tmp_path_factory):
     return run
 
 
+# the arguments nearest to multiples of pi/2, by continued fractions (2^-54 to 2^-60 away)
+NEAREST = np.array([float.fromhex(h) for h in ("0x1.921fb54442d18p+0", "0x1.6c6cbc45dc8dep+5", "0x1.6c6cbc45dc8dep+9",
+                                               "0x1.39c6fd67805a7p+18", "0x1.9eb7148f354d6p+20", "0x1.b951f1572eba5p+23",
+                                               "0x1.b951f1572eba5p+25")])
+
+
 def _arguments(seed, n=40000):
     rng = np.random.default_rng(seed)
-    near = rng.integers(-600000, 600001, n) * (np.pi / 2) * (1 + rng.standard_normal(n) * 2.0 ** rng.integers(-52, -3, n))
-    return np.concatenate([rng.uniform(-r, r, n) for r in (0.8, 10.0, 1e3, 3e4, 2.0 ** 20)] +
-                          [near, 10.0 ** rng.uniform(-300, 0, n), [np.pi / 4, np.pi / 2, np.pi, 2.0 ** 20, -2.0 ** 20]])
+    near = rng.integers(-600000, 600001, n) * 2.0 ** rng.choice([0, 5], n) * (np.pi / 2) * (1 + rng.standard_normal(n) * 2.0 ** rng.integers(-52, -3, n))
+    return np.concatenate([rng.uniform(-r, r, n) for r in (0.8, 10.0, 1e3, 3e4, 2.0 ** 20, 2.0 ** 26)] +
+                          [near, 10.0 ** rng.uniform(-300, 0, n), [np.pi / 4, np.pi / 2, np.pi, 2.0 ** 20, -2.0 ** 20, 2.0 ** 26, -2.0 ** 26],
+                           NEAREST, np.nextafter(NEAREST, 0.0), np.nextafter(NEAREST, np.inf)])
 
 
 def test_reduced_sincos_error(reduced):
@@ -70,7 +77,7 @@ def test_reduced_sincos_zeros(reduced):
 @pytest.mark.gpu
 def test_device_sincos_has_the_host_bits(cuda, reduced):
     """The pair, either of the two alone and the partials, on both engines;
-    past 2^20 and for infinities and NaN the library's values."""
+    past 2^26 and for infinities and NaN the library's values."""
     import torch
     import casadi_amd as ca
     from casadi_amd.hip import HipTape
@@ -78,7 +85,7 @@ def test_device_sincos_has_the_host_bits(cuda, reduced):
     fs = {"pair": [ca.sin(x), ca.cos(x)], "sin": [ca.sin(x)], "cos": [ca.cos(x)]}
     v = _arguments(4, 5000)
     hs, hc = reduced(v)
-    big = np.array([2.0 ** 20 * 1.5, -1e12, 1e300, np.inf, -np.inf, np.nan])
+    big = np.array([2.0 ** 26 * 1.5, -1e12, 1e300, np.inf, -np.inf, np.nan])
     X = torch.tensor(np.concatenate([v, big])[None, :], device="cuda")
     one = torch.ones_like(X)
     print(f"[case] sincos n={X.shape[1]}", flush=True)
